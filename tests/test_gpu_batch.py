@@ -1,0 +1,186 @@
+"""GPU parity of the batches that take more rows than one launch of vs_sample_kernel holds (csrc/vs_batch.hip): the
+streaming pass, the finish from the lists and the open rows, against the NumPy oracle. B = 70 and 130 rows of 8192 and
+more logits always go that way (at most 64 rows fit one launch of the other kernel); 130 rows also use the second half
+of the workspace rows and the second launch of a batch."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import draft_ref as DR
+from oracle import sampler_ref as S
+from parity import check_sample
+from volundr_amd import DeviceSamplers, Sampler, ops, sample_batch, topk_batch
+from volundr_amd.session import Sampling
+
+pytestmark = pytest.mark.gpu
+
+
+def rows_on(dev, x, dtype, pad):
+    """x as a device view whose row stride is V + pad elements."""
+    B, V = x.shape
+    t = torch.empty(B, V + pad, dtype=dtype, device=dev)[:, :V]
+    t.copy_(torch.from_numpy(x).to(dev))
+    return t, t.float().cpu().numpy()
+
+
+def check(dev, x, ps, u, hists=None, dtype=torch.float32, pad=0, pairs=False, label="", max_excused=None):
+    xt, xr = rows_on(dev, x, dtype, pad)
+    print(f"[{label}] B={x.shape[0]} V={x.shape[1]} {dtype} pad={pad} pairs={pairs}", flush=True)
+    out = sample_batch(xt, ps, u, hists, hist_pairs=pairs)
+    torch.cuda.synchronize()
+    refs = [S.sample(xr[i], ps[i], float(u[i]), S.counts_from_history(hists[i]) if hists is not None else {})
+            for i in range(x.shape[0])]
+    check_sample(out, refs, label, max_excused)
+    return out, refs
+
+
+def mixed_params(rng, n, V):
+    out = []
+    for _ in range(n):
+        sp = Sampling(temperature=float(rng.choice([0.0, 0.6, 1.0, 1.0, 1.6])),
+                      top_k=int(rng.choice([0, 0, 0, 1, 20, 64, 65, 128, 256, 257, 300])),
+                      top_p=float(rng.choice([1.0, 0.95, 0.8, 0.3])), min_p=float(rng.choice([0.0, 0.0, 0.05, 0.5])),
+                      repetition_penalty=float(rng.choice([1.0, 1.1, 1.3])),
+                      presence_penalty=float(rng.choice([0.0, 0.3])), frequency_penalty=float(rng.choice([0.0, 0.1])))
+        if rng.random() < 0.3:
+            sp.logit_bias = [(int(t), float(b)) for t, b in zip(rng.integers(0, V, 5), rng.uniform(-4, 4, 5))]
+        if rng.random() < 0.3:
+            sp.suppress_tokens = [0, int(rng.integers(0, V)), V - 1]
+        if rng.random() < 0.3:
+            sp.min_new_tokens, sp.stop_token_ids = 5, [1, V - 2]
+        out.append(sp)
+    return out
+
+
+# a tile is 8192 or 16384 positions: one whole tile, a few logits in the next, several; rows off the 16-byte lines
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,V,pad", [(70, 8192, 0), (70, 8195, 1), (130, 16391, 0), (66, 24577, 7), (130, 16384, 8)])
+def test_mixed_rows(dev, B, V, pad, dtype):
+    rng = np.random.default_rng(V + pad)
+    scale = rng.choice([0.05, 0.3, 1.0, 3.0, 6.0], size=(B, 1))
+    x = (rng.standard_normal((B, V)) * scale).astype(np.float32)
+    hists = [rng.integers(0, V, size=int(rng.integers(0, 2500))) for _ in range(B)]
+    check(dev, x, mixed_params(rng, B, V), rng.random(B), hists, dtype, pad, pairs=bool(pad % 2 == 0),
+          label=f"batch mix {B}x{V}+{pad}")
+
+
+def odd_rows(rng, V):
+    """Rows that lists, bounds and value bins find hard."""
+    n = lambda s: (rng.standard_normal(V) * s).astype(np.float32)  # noqa: E731
+    rows = [np.zeros(V, np.float32), np.full(V, -3.5, np.float32), np.round(n(1.0)), np.round(n(3.0) * 2) / 2]
+    few = np.full(V, -np.inf, np.float32)
+    few[rng.choice(V, 40, replace=False)] = n(2.0)[:40]
+    one = np.full(V, -np.inf, np.float32)
+    one[V - 1] = 1.0
+    none = np.full(V, -np.inf, np.float32)
+    nan = n(2.0)
+    nan[V // 3] = np.nan
+    inf = n(2.0)
+    inf[V // 2] = np.inf
+    low = n(1.0)
+    low[:700] += 12.0 + rng.random(700).astype(np.float32)  # the largest logits all in one chunk
+    huge = n(1.0)
+    huge[5], huge[V - 5] = 2e38, -2e38
+    half = n(1.0)
+    half[::2] = -np.inf
+    zero = n(1e-3)
+    zero[zero < 0] = -0.0
+    return rows + [few, one, none, nan, inf, low, huge, half, zero]
+
+
+@pytest.mark.parametrize("pad", [0, 3])
+@pytest.mark.parametrize("sp", [dict(top_k=20), dict(top_k=200, top_p=0.9), dict(top_p=0.9), dict(), dict(min_p=0.05),
+                                dict(top_p=0.95, min_p=0.01, temperature=0.7), dict(temperature=0.0),
+                                dict(top_k=700), dict(min_p=1.0)], ids=str)
+def test_odd_rows(dev, sp, pad):
+    rng = np.random.default_rng(7 + pad)
+    V = 8192 + 40
+    base = odd_rows(rng, V)
+    x = np.stack((base * 6)[:70])
+    # equal masses have draw boundaries at multiples of 1 / n: keep the draws off them
+    u = (np.floor(rng.random(70) * 4000) + 0.37) / 4000
+    with np.errstate(all="ignore"):
+        check(dev, x, [Sampling(**sp)] * 70, u, pad=pad, label=f"odd rows {sp}")
+
+
+def test_large_counts_and_many_tokens(dev):
+    """Table counts that do not fit the edit words, and a token repeated through a long raw history."""
+    rng = np.random.default_rng(3)
+    B, V = 66, 9000
+    x = (rng.standard_normal((B, V)) * 2).astype(np.float32)
+    ps = [Sampling(top_k=30, repetition_penalty=1.2, frequency_penalty=1e-9, presence_penalty=0.1)] * B
+    u = rng.random(B)
+    tables = [{int(np.argsort(-x[r])[0]): (1 << 28) + 5, int(np.argsort(-x[r])[1]): 3, 7: (1 << 30)} for r in range(B)]
+    xt = torch.from_numpy(x).to(dev)
+    out = sample_batch(xt, ps, u, tables, hist_pairs=True)
+    check_sample(out, [S.sample(x[r], ps[r], float(u[r]), tables[r]) for r in range(B)], "large counts")
+    hists = [np.concatenate([np.full(20000, int(np.argmax(x[r]))), rng.integers(0, V, 700)]) for r in range(B)]
+    check(dev, x, ps, u, hists, label="repeated token", max_excused=1)
+
+
+def test_state_rows(dev):
+    """70 requests with their state on the device: draws, accepted tokens, stop masks and forced rows over steps."""
+    V, B = 8200, 70
+    rng = np.random.default_rng(5)
+    sps = mixed_params(rng, B, V)
+    for i, sp in enumerate(sps):
+        sp.seed = 1000 + i
+    ds = DeviceSamplers([Sampler(sp, vocab_valid=V - 8) for sp in sps], V, hist_cap=64, device=dev)
+    state = [(S.seed_state(1000 + i), [], 0) for i in range(B)]
+    for step in range(4):
+        print(f"[batch state] step {step}", flush=True)
+        x = (rng.standard_normal((B, V)) * 2.5).astype(np.float32)
+        res = ds.step(torch.from_numpy(x).to(dev))
+        refs, nxt = [], []
+        for i, sp in enumerate(sps):
+            rs, u = S.xorshift64s_next(state[i][0])
+            r = S.choose(x[i], sp, V - 8, u, state[i][1])
+            refs.append(r)
+            nxt.append((rs if r.kind == "sample" else state[i][0], state[i][1] + [res.ids[i]], state[i][2] + 1))
+        check_sample(res.out, refs, f"batch state step {step}")
+        state = nxt
+    st = ds.host_state()
+    for i in range(B):
+        assert int(st[i]["rng"]) == state[i][0] and int(st[i]["produced"]) == 4
+        assert ds.history(i) == state[i][1]
+
+
+@pytest.mark.parametrize("k", [1, 16, 64])
+def test_top_lists(dev, k):
+    rng = np.random.default_rng(k)
+    V = 8192 + 24
+    x = np.stack((odd_rows(rng, V) * 6)[:70])
+    xt = torch.from_numpy(x).to(dev)
+    ids, vals = topk_batch(xt, k)
+    ids, vals = ids.cpu().numpy(), vals.cpu().numpy()
+    for r in range(70):
+        ri, rv = DR.topk_sorted(x[r], k)
+        assert np.array_equal(ids[r], ri), (k, r)
+        assert np.array_equal(vals[r], rv), (k, r)
+
+
+def test_graph_replays(dev):
+    """The three launches captured: every replay on refilled logits equals the eager call."""
+    rng = np.random.default_rng(9)
+    B, V = 70, 16500
+    sps = mixed_params(rng, B, V)
+    rows = ops.pack_rows(sps, rng.random(B), V).to(dev)
+    xs = [torch.from_numpy((rng.standard_normal((B, V)) * s).astype(np.float32)).to(dev) for s in (0.2, 2.0, 5.0)]
+    x = xs[0].clone()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        call = ops.PreparedSample([x], rows)
+        call()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        call()
+    for i in (1, 2, 0, 1):
+        x.copy_(xs[i])
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        got = call.out.block.clone()
+        want = ops.sample_rows(xs[i], rows).block
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), i

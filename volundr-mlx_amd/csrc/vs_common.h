@@ -246,6 +246,25 @@ __device__ __forceinline__ T wave_scan(T v) {
   return v;
 }
 
+// Wave reductions whose result every lane gets through one readlane: the steps of wave_scan (one DPP instruction each),
+// the total in lane 63. About a third of the instructions of the butterflies above.
+__device__ __forceinline__ float wave_max_dpp(float v) {
+  auto step = [](float a, uint32_t b) { return fmaxf(a, __uint_as_float(b)); };
+  const uint32_t id = 0xFF800000u;  // -inf
+  v = step(v, dpp32<0x111>(id, __float_as_uint(v)));
+  v = step(v, dpp32<0x112>(id, __float_as_uint(v)));
+  v = step(v, dpp32<0x114>(id, __float_as_uint(v)));
+  v = step(v, dpp32<0x118>(id, __float_as_uint(v)));
+  v = step(v, dpp32<0x142, 0xA>(id, __float_as_uint(v)));
+  v = step(v, dpp32<0x143, 0xC>(id, __float_as_uint(v)));
+  return lane_bcast(v, WAVE - 1);
+}
+__device__ __forceinline__ float wave_min_dpp(float v) { return -wave_max_dpp(-v); }
+template <typename T>
+__device__ __forceinline__ T wave_sum_dpp(T v) {
+  return lane_bcast(wave_scan(v), WAVE - 1);
+}
+
 // Wave-aggregated append: lanes with `pred` get consecutive slots of *counter (an LDS counter), with one atomic per
 // wave instead of one per lane (same-address atomics serialise). Works on LDS or device counters. Returns the
 // slot, or -1.

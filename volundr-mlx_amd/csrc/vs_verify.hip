@@ -497,6 +497,193 @@ __global__ __launch_bounds__(VNT) void vs_verify_kernel(VerifyArgs A) {
   VS_TR_FLUSH(A);
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Blocks of more rows than one launch of vs_verify_kernel holds (its finishers wait for workgroups of their launch, so a
+// launch holds what is resident): one launch over all rows that leaves a partial per workgroup, then one that merges them.
+// What bounds the pass: the logits' stream (2 bytes a bf16 logit) and, close behind, the vector instructions, about ten
+// per logit (one widening kept for both sweeps, the maximum, a check for NaN and infinities, three and a quarter-rate
+// exponential for the sum; the maximum's place by one compare per logit up to where it is found). Eight
+// 16-byte loads per lane, all in flight. 272 rows of V = 248320 bf16 (135 MB): 32 us (4.2 TB/s
+// from the call to its end), 54 in four launches of vs_verify_kernel. f32 keeps 32 logits per lane: 64 of them spill.
+// ---------------------------------------------------------------------------------------------------------------
+constexpr int VSKEY = 5, VSSUM = 6;  // words of a partial slot that hold a workgroup's key and sum (vs_verify_kernel's
+                                     // own words, with their tags and epoch, are left alone)
+constexpr int VMW = 16;              // waves of the merge workgroup
+__host__ __device__ constexpr int vs_lane_logits(int dtype) { return dtype == VS_F32 ? 32 : 64; }  // eight 16-byte loads
+
+template <int DT>
+__global__ __launch_bounds__(VNT, 4) void vs_verify_stream_kernel(VerifyArgs A) {
+  typedef VTraits<DT> TR;
+  constexpr int VEC = TR::VEC, NV = VNF, VSE = NV * VEC, ES = 16 / VEC;
+  static_assert(VSE == vs_lane_logits(DT), "logits per lane");
+  __shared__ u64 wkey[VNW];
+  __shared__ double wsum[VNW];
+  __shared__ float wmx[VNW];
+  const int t = threadIdx.x, wv = t / WAVE, ln = lane_id();
+  const int G = A.G, row = (int)blockIdx.x / G, g = (int)blockIdx.x - row * G;
+  // positions [p0, p1) counted from the 16-byte line the row's first logit lies in (mis logits before it)
+  const char* rowb = (const char*)A.logits + (int64_t)row * A.ld * ES;
+  const int mis = (int)((uintptr_t)rowb & 15) / ES;
+  const char* line = rowb - mis * ES;
+  const int p0 = g * A.CH, p1 = max(p0, min(A.vv + mis, p0 + A.CH));
+  // places outside the chunk read as the lowest finite value: they add nothing to a sum and no NaN to the check below
+  uint4 rv[NV];
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    const int p = p0 + (u * VNT + t) * VEC;
+    constexpr uint32_t LOW = TR::NEG_INF_WORD - (DT == VS_F32 ? 1u : 0x00010001u);
+    rv[u] = make_uint4(LOW, LOW, LOW, LOW);
+    if (p >= mis && p + VEC <= p1) rv[u] = *(const uint4*)(line + (int64_t)p * ES);
+  }
+  float x[VSE];
+#pragma unroll
+  for (int u = 0; u < NV; ++u)
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) x[u * VEC + q] = TR::get(rv[u], q);
+  if (p0 < mis || ((p1 & (VEC - 1)) != 0 && p1 == A.vv + mis)) {  // the row's first and last word
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const int p = p0 + (u * VNT + t) * VEC;
+      if (p < p1 && !(p >= mis && p + VEC <= p1)) {
+#pragma unroll
+        for (int q = 0; q < VEC; ++q)
+          if (p + q >= mis && p + q < p1) x[u * VEC + q] = TR::one(line, p + q);
+      }
+    }
+  }
+  float best = -__builtin_inff(), z0 = 0.0f, z1 = 0.0f;
+#pragma unroll
+  for (int i = 0; i < VSE; i += 2) {
+    best = max3f(best, x[i], x[i + 1]);
+    z0 = __builtin_fmaf(x[i], 0.0f, z0);  // NaN for a NaN or an infinity
+    z1 = __builtin_fmaf(x[i + 1], 0.0f, z1);
+  }
+  const float L2E = 1.44269504088896340736f;
+  const int i0 = p0 - mis + t * VEC;  // the id of the lane's first logit
+  u64 key = 0;
+  double se = 0.0;
+  const float m = wave_max_dpp(best);
+  constexpr float LOWEST = DT == VS_F16 ? -60000.0f : -1e38f;  // a maximum below it could be a place outside the chunk
+  float mw = m;  // the wave's largest finite logit
+  if (__builtin_expect(!__any(!(z0 + z1 == 0.0f)) && m > LOWEST, 1)) {
+    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < VSE; ++i) a[i % 4] += __builtin_amdgcn_exp2f((x[i] - m) * L2E);
+    se = wave_sum_dpp(((double)a[0] + (double)a[1]) + ((double)a[2] + (double)a[3]));
+    // the first place of the maximum: the first vector round any lane has it in, there the first lane, its first place
+    bool found = false;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      if (found) break;
+      bool hit = false;
+#pragma unroll
+      for (int q = 0; q < VEC; ++q) hit |= x[u * VEC + q] == m;
+      const unsigned long long hm = __ballot(hit);
+      if (hm) {
+        int at = 0;
+#pragma unroll
+        for (int q = VEC - 1; q >= 0; --q) at = x[u * VEC + q] == m ? q : at;
+        const int L = __ffsll((long long)hm) - 1;
+        key = amkey64(m, (uint32_t)lane_bcast(i0 + u * VNT * VEC + at, L));
+        found = true;
+      }
+    }
+  } else if (p0 + wv * WAVE * VEC < p1) {  // a NaN or an infinity: element by element (np.argmax's order, NaN first)
+    mw = -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < VSE; ++i) {
+      const int id = i0 + (i / VEC) * VNT * VEC + i % VEC;
+      if (id >= 0 && id < p1 - mis) {
+        const u64 k = amkey64(x[i], (uint32_t)id);
+        key = k > key ? k : key;
+        if (is_finite(x[i])) mw = x[i] > mw ? x[i] : mw;
+      }
+      if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // keeps the unrolled tests from taking all the registers
+    }
+    key = wave_max(key);
+    mw = wave_max_dpp(mw);
+    if (is_finite(mw)) {
+      float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int i = 0; i < VSE; ++i) {
+        const int id = i0 + (i / VEC) * VNT * VEC + i % VEC;
+        const bool in = id >= 0 && id < p1 - mis && is_finite(x[i]);
+        a[i % 4] += __builtin_amdgcn_exp2f(in ? (x[i] - mw) * L2E : -__builtin_inff());
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      se = wave_sum_dpp(((double)a[0] + (double)a[1]) + ((double)a[2] + (double)a[3]));
+    }
+  } else {  // nothing of the chunk for this wave
+    mw = -__builtin_inff();
+  }
+  if (ln == 0) {
+    wkey[wv] = key;
+    wsum[wv] = se;
+    wmx[wv] = mw;
+  }
+  __syncthreads();
+  if (t == 0) {
+    u64 k = wkey[0];
+    float M = wmx[0];
+#pragma unroll
+    for (int i = 1; i < VNW; ++i) {
+      k = wkey[i] > k ? wkey[i] : k;
+      M = wmx[i] > M ? wmx[i] : M;
+    }
+    double S = 0.0;
+#pragma unroll
+    for (int i = 0; i < VNW; ++i)
+      S += wsum[i] > 0.0 ? wsum[i] * (double)__builtin_amdgcn_exp2f((wmx[i] - M) * L2E) : 0.0;
+    VPart* pp = (VPart*)(A.ws + 16 * VRMAX) + (size_t)row * VGMAX + g;
+    pp->w[VSKEY] = k;
+    pp->w[VSSUM] = (u64)__double_as_longlong(S);
+  }
+}
+
+// One workgroup per request: a wave per row merges the row's partials, then the accept length (specdec.py:326-327). A
+// partial's maximum is its key's value; a key of a NaN or an infinity makes the logprob 0 whatever the sums are.
+__global__ __launch_bounds__(VMW * WAVE) void vs_verify_merge_kernel(VerifyArgs A) {
+  extern __shared__ int32_t tok[];  // [T]
+  const int req = blockIdx.x, wv = threadIdx.x / WAVE, ln = lane_id();
+  const int nslots = A.G;
+  const float L2E = 1.44269504088896340736f;
+  for (int r = wv; r < A.T; r += (int)blockDim.x / WAVE) {
+    const int64_t row = (int64_t)req * A.T + r;
+    const VPart* pp = (const VPart*)(A.ws + 16 * VRMAX) + (size_t)row * VGMAX + (ln < nslots ? ln : 0);
+    const u64 k = ln < nslots ? pp->w[VSKEY] : (u64)0;
+    const double e = __longlong_as_double((long long)pp->w[VSSUM]);
+    const float v = k ? key_value(k) : -__builtin_inff();
+    const bool in = ln < nslots && is_finite(v) && e > 0.0;
+    const u64 bam = wave_max(k);
+    const float M = wave_max_dpp(in ? v : -__builtin_inff());
+    const double S = wave_sum_dpp(in ? e * (double)__builtin_amdgcn_exp2f((v - M) * L2E) : 0.0);
+    if (ln == 0) {
+      const int32_t id = bam ? (int32_t)key_index(bam) : -1;
+      tok[r] = id;
+      A.out_argmax[row] = id;
+      if (A.out_lp) {
+        const float xj = am_is_nan(bam) ? __builtin_nanf("") : key_value(bam);
+        A.out_lp[row] =
+            (is_finite(xj) && S > 0.0) ? (float)((double)xj - ((double)M + (double)log1pf((float)(S - 1.0)))) : 0.0f;
+      }
+    }
+  }
+  __syncthreads();
+  if (wv != 0) return;
+  const int32_t* dr = A.drafts + (size_t)req * (A.T - 1);
+  int nacc = 0;
+  for (int base = 0; base < A.T - 1; base += WAVE) {
+    const int i = base + ln;
+    const unsigned long long mb = __ballot(i >= A.T - 1 || dr[i] != tok[i]);
+    if (mb) {
+      nacc += __ffsll((long long)mb) - 1;
+      break;
+    }
+    nacc += WAVE;
+  }
+  if (ln == 0) A.out_accept[req] = nacc;
+}
+
 }  // namespace vs
 
 using namespace vs;
@@ -568,6 +755,31 @@ extern "C" int vs_verify_greedy(const void* logits, int dtype, int B, int T, int
   const int cap = per_cu * dv->cus;
   int rpl = cap / G;
   if (rpl < 1) rpl = 1;
+  // More rows than that: the pass over all of them and the merge, two launches whatever the number of rows. A chain of
+  // launches, each with its own start, tail and finish, took for 272 rows of V = 248320 bf16 53.8 us, the two take 32.3;
+  // V = 163840: 37.0 and 21.5 in bf16, 54.6 and 35.8 in f32. In one launch vs_verify_kernel is the better one (17 rows of
+  // V = 163840 bf16: 6.8 us against 8.5; 102 rows 13.5 against 13.4), except where rows are unaligned, since it reads
+  // those element by element: 17 rows of ld = 163843 9.9 against 8.8, 68 rows 19.9 against 12.4, 68 of 50003 f16 11.2
+  // against 10.1, but 34 of those 8.7 against 9.7. Hence the line at 2 M logits.
+  const int es = 16 / VEC;
+  const int span = vocab_valid + (ld % VEC == 0 ? (int)((uintptr_t)logits % 16) / es : VEC - 1);
+  const int tile = VNT * vs_lane_logits(dtype), gs = (span + tile - 1) / tile;
+  const bool many = R > rpl || (!a.vec_ok && (int64_t)R * vocab_valid >= (2 << 20));
+  if (many && gs <= VGMAX && (uintptr_t)logits % es == 0) {
+    a.CH = ((span + gs - 1) / gs + VEC - 1) / VEC * VEC;
+    a.G = (span + a.CH - 1) / a.CH;
+    a.row0 = 0;
+    void* kargs[] = {&a};
+    const void* sfn = dtype == VS_F32    ? (const void*)vs_verify_stream_kernel<VS_F32>
+                      : dtype == VS_BF16 ? (const void*)vs_verify_stream_kernel<VS_BF16>
+                                         : (const void*)vs_verify_stream_kernel<VS_F16>;
+    hipError_t e = hipLaunchKernel(sfn, dim3((unsigned)(R * a.G)), dim3(VNT), kargs, 0, (hipStream_t)stream);
+    const int waves = T < VMW ? T : VMW;
+    if (e == hipSuccess)
+      e = hipLaunchKernel((const void*)vs_verify_merge_kernel, dim3((unsigned)B), dim3((unsigned)(waves * WAVE)), kargs,
+                          (size_t)T * 4, (hipStream_t)stream);
+    return e == hipSuccess ? VS_OK : hip_fail(e, "vs_verify_greedy: launch");
+  }
   for (int r0 = 0; r0 < R; r0 += rpl) {
     const int n = (R - r0) < rpl ? (R - r0) : rpl;
     a.row0 = r0;

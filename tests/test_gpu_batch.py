@@ -118,6 +118,34 @@ def test_large_counts_and_many_tokens(dev):
     check(dev, x, ps, u, hists, label="repeated token", max_excused=1)
 
 
+@pytest.mark.parametrize("pairs", [False, True])
+def test_lengths_of_the_edit_lists(dev, pairs):
+    """Tables, histories, masks and biases that end at, before and past what a lane loads ahead (512 ids of a list, 2048
+    table entries, 4096 raw tokens, then rounds of 12288), with the row's largest logits among their ids."""
+    rng = np.random.default_rng(9)
+    B, V = 66, 33000
+    x = (rng.standard_normal((B, V)) * 2).astype(np.float32)
+    top = np.argsort(-x, axis=1)[:, :4000]
+    lens = [1, 3, 511, 512, 513, 2047, 2048, 2049, 4095, 4096, 4103, 16384, 16391, 30000]
+    few = [0, 1, 511, 512, 513, 1100]
+    ps, hists = [], []
+    for r in range(B):
+        n, m = lens[r % len(lens)], few[r % len(few)]
+        ids = np.concatenate([top[r][: min(n, 300)], rng.permutation(V)])  # unique once cut, in an order of no kind
+        ids = ids[np.sort(np.unique(ids, return_index=True)[1])][:n]
+        if not pairs:
+            ids = np.concatenate([ids[: n - n // 3], rng.choice(ids, n // 3)]) if n > 3 else ids
+        hists.append(rng.permutation(ids))
+        sp = Sampling(temperature=0.9, top_k=[40, 0, 64][r % 3], top_p=0.95, repetition_penalty=1.2, presence_penalty=0.2,
+                      frequency_penalty=0.05)
+        if m:
+            sp.suppress_tokens = [int(i) for i in rng.choice(top[r], m, replace=False)]
+            sp.logit_bias = [(int(i), float(b)) for i, b in zip(rng.choice(top[r], m), rng.uniform(-2, 2, m))]
+            sp.min_new_tokens, sp.stop_token_ids = 5, [int(i) for i in rng.choice(top[r], m, replace=False)]
+        ps.append(sp)
+    check(dev, x, ps, rng.random(B), hists, pairs=pairs, pad=3, label="edit lists")
+
+
 def test_state_rows(dev):
     """70 requests with their state on the device: draws, accepted tokens, stop masks and forced rows over steps."""
     V, B = 8200, 70

@@ -310,6 +310,13 @@ int vs_stream_read(const void* p, size_t bytes, int blocks, uint32_t* out, vs_st
  * counterpart in the reference. */
 int vs_xcd_ids(uint32_t* out, int blocks, int threads, vs_stream_t stream);
 
+/* How a batch of B rows that takes more than one launch of the one-launch kernel is split on a device of `cus` CUs
+ * (mis: logits between the 16-byte line and the first logit; ws_bytes: the workspace): a testing hook, host code alone.
+ * out[7]: rows per launch, logits per lane, workgroups per row, positions per workgroup, keys of a workgroup's list at
+ * most, largest top_k finished from the lists, candidates per workgroup of a row without a top-k cut. No counterpart in
+ * the reference. */
+int vs_batch_plan(int dtype, int V, int64_t ld, int mis, int B, size_t ws_bytes, int cus, int* out);
+
 /* Zero a workspace (stream-ordered). */
 int vs_workspace_init(void* ws, size_t bytes, vs_stream_t stream);
 

@@ -1177,7 +1177,8 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   __syncthreads();
   const int nitems = s.misc[0];
   if (nitems == 0) return;
-  // workgroups per row: as many as leave a cluster for every row (top lists: one, no waiting)
+  // workgroups per row: as many as leave a cluster for every row (top lists: one, no waiting); no more rows than
+  // workgroups (batch_plan)
   const int C = A.list_k > 0 ? 1 : max(1, min(CMAX, (int)gridDim.x / nitems));
   const int nb = gridDim.x, b = blockIdx.x;
   const int l = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;  // a cluster's workgroups on one XCD where they fit
@@ -1743,42 +1744,65 @@ static const void* stream_fn(int E) {
   return E == 16 ? (const void*)vs_batch_kernel<DT, 16 / VEC> : (const void*)vs_batch_kernel<DT, 32 / VEC>;
 }
 
-int batch_path(SampleArgs a, int dtype, int B, size_t ws_rows, const DevInfo* dv, hipStream_t stream) {
+// How a batch of B rows is launched on a device of `cus` CUs; mis: logits between the 16-byte line and the first logit.
+struct BatchPlan {
+  int rows;  // rows per launch
+  int E;     // logits per lane of the stream kernel
+  int G;     // its workgroups per row
+  int CH;    // positions per workgroup
+  int kcap;  // keys of a chunk's list at most
+  int kmax;  // largest top_k finished from the lists
+  int nv;    // candidates per chunk of a row without a top-k cut
+};
+static BatchPlan batch_plan(int V, int64_t ld, int dtype, int mis, int B, size_t ws_rows, int cus) {
   const int VEC = dtype == VS_F32 ? 4 : 8;
-  const int nmax = ws_rows >= (size_t)RPL_MAX ? BATCH_ROWS : (int)ws_rows;
-  const int nrows = B < nmax ? B : nmax;
+  BatchPlan p;
+  // The resolve kernel has a workgroup per CU and gives every open row at least one: no more rows than CUs (a device
+  // partition can have fewer than BATCH_ROWS).
+  int nmax = ws_rows >= (size_t)RPL_MAX ? BATCH_ROWS : (int)ws_rows;
+  if (nmax > cus) nmax = cus;
+  p.rows = B < nmax ? B : nmax;
   // positions of a row, counted from the 16-byte line of its first logit (the rows' places in their lines differ
   // unless the stride is a multiple of 16 bytes)
-  const int es = 16 / VEC;
-  const int span = a.V + (a.ld % VEC == 0 ? (int)((uintptr_t)a.logits % 16) / es : VEC - 1);
+  const int span = V + (ld % VEC == 0 ? mis : VEC - 1);
   // Logits per lane. 32 spend fewer instructions per logit and leave the finish kernel half the lists, 16 keep three
   // workgroups on a CU instead of two and give a small batch enough of them. V = 163840 fp32, mixed requests, us per
   // call with 16 / 32: B = 24 26.8 / 27.7, 48 34.3 / 31.7, 96 42.6 / 41.0; the line lies where 32 still fill the CUs
   // one and a half times.
   const int g32 = (span + 32 * SNT - 1) / (32 * SNT), g16 = (span + 16 * SNT - 1) / (16 * SNT);
-  const int E = 2 * nrows * g32 >= 3 * dv->cus || g16 > GMAX ? 32 : 16;
-  int G = E == 32 ? g32 : g16;
-  const int CH = ((span + G - 1) / G + VEC - 1) / VEC * VEC;
-  G = (span + CH - 1) / CH;
-  a.G = G;
-  a.CH = CH;
-  const int per_wave = (G + SNW - 1) / SNW;  // lists a wave of the finish kernel takes, BATCH_NK rounds of 64 keys together
-  a.kcap = (nrows > RPL_MAX ? BIGCAP : KEYS_CAP) / G / WAVE * WAVE;
-  if (a.kcap > BATCH_NK / per_wave * WAVE) a.kcap = BATCH_NK / per_wave * WAVE;
-  a.kmax = a.kcap < KCAP ? a.kcap : KCAP;
+  p.E = 2 * p.rows * g32 >= 3 * cus || g16 > GMAX ? 32 : 16;
+  p.G = p.E == 32 ? g32 : g16;
+  p.CH = ((span + p.G - 1) / p.G + VEC - 1) / VEC * VEC;
+  p.G = (span + p.CH - 1) / p.CH;
+  const int per_wave = (p.G + SNW - 1) / SNW;  // lists a wave of the finish kernel takes, BATCH_NK rounds of 64 keys together
+  p.kcap = (p.rows > RPL_MAX ? BIGCAP : KEYS_CAP) / p.G / WAVE * WAVE;
+  if (p.kcap > BATCH_NK / per_wave * WAVE) p.kcap = BATCH_NK / per_wave * WAVE;
+  p.kmax = p.kcap < KCAP ? p.kcap : KCAP;
   // candidates per chunk of a row without a top-k cut (a chunk lists about 1.5 times as many): the nucleus of a language
   // model's row is a few hundred logits; 48, 64 and 96 measured within 2% of one another
-  a.NV = a.kcap / 3 / 8 * 8 < 64 ? a.kcap / 3 / 8 * 8 : 64;
-  const void* sfn = dtype == VS_F32 ? stream_fn<VS_F32>(E) : dtype == VS_BF16 ? stream_fn<VS_BF16>(E) : stream_fn<VS_F16>(E);
+  p.nv = p.kcap / 3 / 8 * 8 < 64 ? p.kcap / 3 / 8 * 8 : 64;
+  return p;
+}
+
+int batch_path(SampleArgs a, int dtype, int B, size_t ws_rows, const DevInfo* dv, hipStream_t stream) {
+  const int es = dtype == VS_F32 ? 4 : 2;
+  const BatchPlan p = batch_plan(a.V, a.ld, dtype, (int)((uintptr_t)a.logits % 16) / es, B, ws_rows, dv->cus);
+  a.G = p.G;
+  a.CH = p.CH;
+  a.kcap = p.kcap;
+  a.kmax = p.kmax;
+  a.NV = p.nv;
+  const void* sfn =
+      dtype == VS_F32 ? stream_fn<VS_F32>(p.E) : dtype == VS_BF16 ? stream_fn<VS_BF16>(p.E) : stream_fn<VS_F16>(p.E);
   const void* rfn = dtype == VS_F32    ? (const void*)vs_resolve_kernel<VS_F32>
                     : dtype == VS_BF16 ? (const void*)vs_resolve_kernel<VS_BF16>
                                        : (const void*)vs_resolve_kernel<VS_F16>;
   const void* ffn = (const void*)vs_finish_kernel;
-  for (int r0 = 0; r0 < B; r0 += nmax) {
+  for (int r0 = 0; r0 < B; r0 += p.rows) {
     a.row0 = r0;
-    a.B = (B - r0) < nmax ? (B - r0) : nmax;
+    a.B = (B - r0) < p.rows ? (B - r0) : p.rows;
     void* kargs[] = {&a};
-    hipError_t e = hipLaunchKernel(sfn, dim3((unsigned)(a.B * G)), dim3(SNT), kargs, stream_lds(E * SNT), stream);
+    hipError_t e = hipLaunchKernel(sfn, dim3((unsigned)(a.B * p.G)), dim3(SNT), kargs, stream_lds(p.E * SNT), stream);
     if (e == hipSuccess) e = hipLaunchKernel(ffn, dim3((unsigned)a.B), dim3(SNT), kargs, 0, stream);
     // one workgroup per CU: all resident, so that a cluster's waits end
     if (e == hipSuccess) e = hipLaunchKernel(rfn, dim3((unsigned)dv->cus), dim3(SNT), kargs, RESOLVE_LDS, stream);
@@ -1788,3 +1812,13 @@ int batch_path(SampleArgs a, int dtype, int B, size_t ws_rows, const DevInfo* dv
 }
 
 }  // namespace vs
+
+extern "C" int vs_batch_plan(int dtype, int V, int64_t ld, int mis, int B, size_t ws_bytes, int cus, int* out) {
+  if (!out || V < 1 || ld < V || mis < 0 || B < 1 || cus < 1 || ws_bytes < vs::ROW_WS ||
+      (dtype != VS_F32 && dtype != VS_BF16 && dtype != VS_F16))
+    return vs::fail(VS_EINVAL, "vs_batch_plan: bad arguments");
+  const vs::BatchPlan p = vs::batch_plan(V, ld, dtype, mis, B, ws_bytes / vs::ROW_WS, cus);
+  const int v[] = {p.rows, p.E, p.G, p.CH, p.kcap, p.kmax, p.nv};
+  for (int i = 0; i < 7; ++i) out[i] = v[i];
+  return VS_OK;
+}

@@ -55,7 +55,8 @@ EXPORTS = ("vs_sample_batch", "vs_sample_batch_state", "vs_state_fold", "vs_samp
            "vs_verify_workspace_bytes", "vs_topk_batch", "vs_draft_walk", "vs_draft_propose",
            "vs_draft_workspace_bytes", "vs_lmhead_verify_greedy", "vs_lmhead_workspace_bytes", "vs_lmhead_sample",
            "vs_lmhead_sample_workspace_bytes", "vs_set_spin_limit", "vs_workspace_init", "vs_last_error", "vs_version",
-           "vs_sample_batch_noalloc", "vs_sample_noalloc_scratch_bytes", "vs_launch_floor", "vs_stream_read", "vs_xcd_ids", "vs_set_cooperative", "vs_set_debug")
+           "vs_sample_batch_noalloc", "vs_sample_noalloc_scratch_bytes", "vs_launch_floor", "vs_stream_read", "vs_xcd_ids", "vs_set_cooperative",
+           "vs_set_debug", "vs_batch_plan")
 
 _lib = None
 
@@ -99,6 +100,8 @@ def load():
     L.vs_launch_floor.restype = i32
     L.vs_xcd_ids.argtypes = [vp, i32, i32, vp]
     L.vs_xcd_ids.restype = i32
+    L.vs_batch_plan.argtypes = [i32, i32, i64, i32, i32, sz, i32, vp]
+    L.vs_batch_plan.restype = i32
     L.vs_set_debug.argtypes = [ctypes.c_uint]
     L.vs_set_debug.restype = i32
     L.vs_set_cooperative.argtypes = [i32]

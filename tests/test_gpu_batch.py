@@ -9,7 +9,7 @@ import torch
 from oracle import draft_ref as DR
 from oracle import sampler_ref as S
 from parity import check_sample
-from volundr_amd import DeviceSamplers, Sampler, ops, sample_batch, topk_batch
+from volundr_amd import DeviceSamplers, Sampler, _lib, ops, sample_batch, topk_batch
 from volundr_amd.session import Sampling
 
 pytestmark = pytest.mark.gpu
@@ -212,3 +212,22 @@ def test_graph_replays(dev):
         want = ops.sample_rows(xs[i], rows).block
         torch.cuda.synchronize()
         assert torch.equal(got, want), i
+
+
+def test_tag_words_left_alone(dev):
+    """The words that hold the other kernel's tags keep what it left there, whatever a large batch does: that kernel
+    takes a partial for this call's own by them."""
+    rng = np.random.default_rng(12)
+    B, V = 70, 8200
+    row = _lib.load().vs_sample_workspace_bytes(1, V)
+    x = torch.from_numpy((rng.standard_normal((B, V)) * 2).astype(np.float32)).to(dev)
+    ps = mixed_params(rng, B, V)
+    sample_batch(x, ps, rng.random(B))  # the workspace is as large as it gets
+    sample_batch(x[:16], ps[:16], rng.random(16))
+    ws = ops.workspace(dev, 64 * row)
+    at = torch.tensor([r * row + 128 + 96 * g + 20 + i for r in range(64) for g in range(64) for i in range(4)], device=dev)
+    before = ws[at].clone()
+    print("[tags] 70 rows", flush=True)
+    sample_batch(x, ps, rng.random(B))
+    torch.cuda.synchronize()
+    assert torch.equal(ws[at], before)

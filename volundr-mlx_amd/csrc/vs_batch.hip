@@ -34,7 +34,8 @@ constexpr int CMAX = 32;                 // workgroups per open row at most
 
 // Workspace of a launch's row r: workspace rows hold two each. Row r < RPL_MAX uses the part and cand areas of
 // workspace row r, row r >= RPL_MAX the gather and big areas of workspace row r - RPL_MAX (areas whose contents no call
-// relies on). The open flags sit in the control blocks' lines, after RowCtl: those of rows [56 k, 56 k + 56) in
+// relies on; of a partial all but the word `pad`, by whose tags vs_sample_kernel tells this call's partials from what
+// earlier ones left). The open flags sit in the control blocks' lines, after RowCtl: those of rows [56 k, 56 k + 56) in
 // workspace row k. Nothing here has to be zero when a call starts.
 enum { ROW_DONE = 0, ROW_FLAT = 1, ROW_ANY = 2 };  // open flag: finished, left to the flat or to the general method
 constexpr size_t OFF_OPEN = 64;
@@ -56,11 +57,12 @@ struct OpenRow {
   float xmax, xmin;  // the largest and smallest of them
   uint32_t bar;      // arrivals at the cluster's barriers
   uint32_t gcnt;     // gathered keys
-  uint32_t pad;
+  uint32_t tag;      // the first partial's tag word, left alone
   uint32_t cnt[4];   // sums over the cluster: counts
   double mass[4];    // and masses
   u64 amkey;
 };
+static_assert(offsetof(OpenRow, tag) == offsetof(Part, pad) && sizeof(OpenRow) <= sizeof(Part), "the tag words stay");
 // An open row's list area: the mass histogram of the flat method (or the ring of radix histograms), then the keys.
 struct RadixSlot {
   uint32_t cnt[NBIN];
@@ -754,7 +756,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_batch_kernel(SampleArgs A) {
       for (int i = 0; i < SNW; ++i) r += s.sum[i];
       part->nfin = (uint32_t)nf;
       part->kc = (uint32_t)(bad ? 0 : C);
-      part->pad = bad ? L_NONE : L;
+      part->heads[1] = bad ? L_NONE : L;  // (the tag word `pad` is vs_sample_kernel's alone)
       part->heads[0] = ((u64)__float_as_uint(wm) << 32) | __float_as_uint(mn);
       part->se = r;
     }
@@ -832,7 +834,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
   const bool full = cls == CLS_FULL;
   const int k = full ? A.NV : top_k;
   const int cg = ln < G ? (int)pp.kc : 0;           // list ln's length
-  const uint32_t pl = ln < G ? pp.pad : 0u;         // its bound
+  const uint32_t pl = ln < G ? (uint32_t)pp.heads[1] : 0u;  // its bound
   const int pn = ln < G ? (int)pp.nfin : 0;
   const float pm = pn ? __uint_as_float((uint32_t)(pp.heads[0] >> 32)) : -__builtin_inff();
   const float pmn = pn ? __uint_as_float((uint32_t)pp.heads[0]) : __builtin_inff();

@@ -259,11 +259,12 @@ int vs_draft_propose(const void* logits, int dtype, int n, int S, int V, int64_t
 size_t vs_draft_workspace_bytes(int n, int S, int V);
 
 /* The inter-workgroup waits of vs_sample_batch / vs_sample_batch_state (row barriers of rows with top-k off or above
- * 256) give up after 200 us (5 ms under a cooperative launch), measured on the GPU's 100 MHz real-time counter, and
- * flag their row VS_OUT_TIMEOUT. A testing hook: a non-zero `polls` also bounds each wait of later plain launches of
+ * 256) give up after 200 us (5 ms under a cooperative launch; 1 ms in batches of more rows than one launch holds, where
+ * rows with flat distributions and rows without a finite logit wait), measured on the GPU's 100 MHz real-time counter,
+ * and flag their row VS_OUT_TIMEOUT. A testing hook: a non-zero `polls` also bounds each wait of later plain launches of
  * the process by that many polls (0 restores the time bound alone), so a tiny limit forces the timeout path, whose
- * rows report VS_OUT_TIMEOUT, commit no request state and leave the workspace zeroed. No counterpart in the
- * reference (its sampler is single-threaded host code). */
+ * rows report VS_OUT_TIMEOUT, commit no request state and leave the workspace fit for the next call. No counterpart in
+ * the reference (its sampler is single-threaded host code). */
 int vs_set_spin_limit(unsigned polls);
 
 /* Testing flags for later calls of the process (0 restores the default behaviour). VS_DEBUG_FORCE_RADIX: rows of

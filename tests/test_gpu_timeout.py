@@ -343,3 +343,90 @@ def test_xcd_split_recovers_with_the_coherent_exchange(dev):
     with pytest.warns(RuntimeWarning, match="device-coherent"):
         got, _ = _debug(_lib.DEBUG_FAKE_XCD_SPLIT, lambda: _sample_checked(x, *args))
     assert (got.ids.cpu().tolist(), got.logprobs.cpu().tolist()) == w
+
+
+# ---------------------------------------------------------------- batches above one launch (csrc/vs_batch.hip)
+def _flat_and_peaked(seed, B=70, V=65536):
+    """Requests whose distributions are flat (rows that a cluster of workgroups finishes, waiting for one another) and
+    top-k and greedy ones (rows that wait for nothing), in turn."""
+    g = np.random.default_rng(seed)
+    x = (g.standard_normal((B, V)) * 0.1).astype(np.float32)
+    kinds = [dict(top_p=0.95), dict(top_k=20), dict(temperature=0.0), dict(temperature=0.7), dict(top_k=64, top_p=0.9)]
+    return x, [Sampling(**kinds[r % 5]) for r in range(B)], [r % 5 in (0, 3) for r in range(B)]
+
+
+def _state(sps, V, dev):
+    ss = []
+    for r, sp in enumerate(sps):
+        s = Sampler(sp, vocab_valid=V, request_id=r)
+        s.rng = 0x2468ACE ^ r
+        ss.append(s)
+    return DeviceSamplers(ss, V, hist_cap=64, device=dev)
+
+
+def test_open_rows_that_give_up_commit_nothing(dev):
+    """A waiting workgroup that gives up ends its row with VS_OUT_TIMEOUT and leaves the request's state; rows that
+    finished without waiting are committed once; the next step is exact."""
+    xn, sps, flat = _flat_and_peaked(3)
+    x, V = torch.from_numpy(xn).to(dev), xn.shape[1]
+    ref, ds = _state(sps, V, dev), _state(sps, V, dev)
+    want = ref.step(x)
+    st_want, st0 = ref.host_state().copy(), ds.host_state().copy()
+    assert not any(f & OUT_TIMEOUT for f in want.flags)
+    print("[timeout] open rows forced", flush=True)
+    out = _forced(lambda: ds.step(x, sync=False))
+    fl, ids, st1 = _flags(out), out.ids.cpu().tolist(), ds.host_state()
+    timed = [bool(f & OUT_TIMEOUT) for f in fl]
+    print(f"[timeout]   flagged {sum(timed)} of {len(fl)}, {sum(flat)} flat", flush=True)
+    assert any(timed) and not any(t and not f for t, f in zip(timed, flat))
+    for r in range(len(fl)):
+        if timed[r]:
+            assert np.array_equal(st1[r], st0[r]), r
+        else:
+            assert ids[r] == want.ids[r] and np.array_equal(st1[r], st_want[r]), r
+    again = _state(sps, V, dev).step(x)
+    assert again.ids == want.ids and again.logprobs == want.logprobs
+
+
+def test_open_rows_retry(dev):
+    """DeviceSamplers.step and sample_rows_for repeat such rows under a cooperative launch (the other kernel, on the
+    workspace the batch route has used)."""
+    from volundr_amd.sampler import sample_rows_for
+
+    xn, sps, _ = _flat_and_peaked(4)
+    x, V = torch.from_numpy(xn).to(dev), xn.shape[1]
+    ref, ds = _state(sps, V, dev), _state(sps, V, dev)
+    want = ref.step(x)
+    print("[timeout] open rows retried, device state", flush=True)
+    got = _forced(lambda: ds.step(x))
+    assert got.ids == want.ids and np.allclose(got.logprobs, want.logprobs, rtol=1e-5, atol=1e-10)
+    assert not any(f & OUT_TIMEOUT for f in got.flags)
+    assert np.array_equal(ds.host_state(), ref.host_state())
+    mk = lambda: [Sampler(sp, vocab_valid=V, request_id=r) for r, sp in enumerate(sps)]  # noqa
+    a, b = mk(), mk()
+    for sa, sb in zip(a, b):
+        sb.rng = sa.rng
+    want_ids = sample_rows_for(x, a)
+    print("[timeout] open rows retried, host state", flush=True)
+    assert _forced(lambda: sample_rows_for(x, b)) == want_ids and [s.rng for s in a] == [s.rng for s in b]
+
+
+def test_exchange_level_leaves_the_route_of_large_batches(dev):
+    """VS_DEBUG_NO_XCD_EXCHANGE (which the retry path sets for good) concerns the kernel of one launch: a large batch
+    gives the same bits by the same route. The route shows in the workspace's open flags, which it alone writes."""
+    xn, sps, _ = _flat_and_peaked(5)
+    x, V = torch.from_numpy(xn).to(dev), xn.shape[1]
+    rows = ops.pack_rows(sps, np.random.default_rng(5).random(len(sps)), V).to(dev)
+    want = ops.sample_rows(x, rows).block.clone()
+    row = _lib.load().vs_sample_workspace_bytes(1, V)
+    ws = ops.workspace(dev, 64 * row)
+
+    def routed():
+        ws[64] = 0xEE  # the first row's open flag
+        out = ops.sample_rows(x, rows).block.clone()
+        torch.cuda.synchronize()
+        return int(ws[64]) != 0xEE, out
+
+    assert routed()[0]
+    on_route, got = _debug(_lib.DEBUG_NO_XCD_EXCHANGE, routed)
+    assert on_route and torch.equal(got, want)

@@ -1246,7 +1246,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   bool ok = true;
   auto barrier = [&]() -> bool {  // every store and atomic of the cluster before it is seen after it
     ++nbar;
-    ok = row_barrier(&o->bar, nbar * (uint32_t)C, 0xFFFFFFFFu, WAIT_TICKS_OPEN, &s.misc[1]);
+    ok = row_barrier(&o->bar, nbar * (uint32_t)C, A.spin_limit, WAIT_TICKS_OPEN, &s.misc[1]);
     return ok;
   };
   Final fin;

@@ -2816,10 +2816,11 @@ static int sample_launch(const void* logits, int dtype, int B, int V, int64_t ld
   // shorter way for up to RB rows unless their mix is unlucky (V = 163840 fp32, us per call here / there: 16 top-k rows
   // 13 / 18, 16 near-flat ones 31 / 48, 16 mixed requests 61 / 26), a chain of launches is not (20 / 64 rows: top-k
   // 27 / 19 and 55 / 22, near-flat 60 / 51 and 127 / 108, mixed requests 140 / 27 and 255 / 37). Rows below 8192
-  // logits give its workgroups too few lanes to bound their lists with. The testing hooks and cooperative launches
-  // concern this kernel's waits, and vs_sample_batch_noalloc's scratch rows are its own.
+  // logits give its workgroups too few lanes to bound their lists with. The testing flags (but the exchange level, which
+  // that route has only one of) and cooperative launches concern this kernel's waits, and vs_sample_batch_noalloc's
+  // scratch rows are its own.
   const size_t ws_rows = ws_bytes / ROW_WS;
-  if (B > RB && V >= 8192 && list_k <= WAVE && rows_cap == RPL_MAX && !coop && !g_debug && !g_spin_limit &&
+  if (B > RB && V >= 8192 && list_k <= WAVE && rows_cap == RPL_MAX && !coop && !(g_debug & ~VS_DEBUG_NO_XCD_EXCHANGE) &&
       (uintptr_t)logits % (16 / VEC) == 0)
     return batch_path(a, dtype, B, ws_rows, dv, (hipStream_t)stream);
   for (int r0 = 0; r0 < B; r0 += RB) {

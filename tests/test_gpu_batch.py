@@ -231,3 +231,49 @@ def test_tag_words_left_alone(dev):
     sample_batch(x, ps, rng.random(B))
     torch.cuda.synchronize()
     assert torch.equal(ws[at], before)
+
+
+def hard_lists(rng, V, n):
+    """n rows whose chunks have more candidates than their lists hold: continuous values, values in steps (thousands of
+    ties at the cut), one value, the largest logits side by side, few finite logits."""
+    rows = []
+    for r in range(n):
+        x = (rng.standard_normal(V) * 2).astype(np.float32)
+        if r % 5 == 1:
+            x = np.round(x * 2) / 2
+        elif r % 5 == 2:
+            x[:] = -1.25 if r % 2 else 0.0
+            x[::7] = -0.0 if r % 2 == 0 else -1.25
+        elif r % 5 == 3:
+            at = int(rng.integers(0, V - 3000))
+            x[at:at + 3000] += 12.0
+        elif r % 5 == 4:
+            x[rng.random(V) < 0.99] = -np.inf
+        rows.append(x)
+    return np.stack(rows)
+
+
+@pytest.mark.parametrize("B,V,pad,dtype", [(20, 248320, 0, torch.bfloat16), (66, 163840, 0, torch.float32),
+                                           (40, 100003, 3, torch.float16), (70, 8192, 0, torch.float32)])
+def test_top_k_above_what_a_bound_lists(dev, B, V, pad, dtype):
+    """top_k up to 256 where the chunks' bounds let more candidates through than a list holds."""
+    rng = np.random.default_rng(B)
+    x = hard_lists(rng, V, B)
+    ps = [Sampling(top_k=int([256, 100, 200, 160, 128, 255, 64][r % 7]), top_p=float([1.0, 0.9][r % 2]), temperature=1.3)
+          for r in range(B)]
+    u = (np.floor(rng.random(B) * 4000) + 0.37) / 4000  # equal masses: draws off the multiples of 1 / n
+    check(dev, x, ps, u, dtype=dtype, pad=pad, label=f"top-k lists {B}x{V}", max_excused=1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [16, 64])
+def test_top_lists_of_tied_values(dev, k, dtype):
+    rng = np.random.default_rng(k)
+    B, V = 32, 100008
+    xt, x = rows_on(dev, hard_lists(rng, V, B), dtype, 0)
+    print(f"[tied lists] k={k} {dtype}", flush=True)
+    ids, vals = topk_batch(xt, k)
+    ids, vals = ids.cpu().numpy(), vals.cpu().numpy()
+    for r in range(B):
+        ri, rv = DR.topk_sorted(x[r], k)
+        assert np.array_equal(ids[r], ri) and np.array_equal(vals[r], rv), (k, r)

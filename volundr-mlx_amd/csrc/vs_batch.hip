@@ -6,15 +6,16 @@
 // launches, each as long as its slowest row. Here
 //   vs_batch_kernel    streams the logits once, a chunk per workgroup in registers, and leaves per chunk a short list:
 //     GREEDY  the first-max key and the log-sum-exp partial;
-//     TOPK    at least its k largest logits, so the row's k largest are in the lists;
+//     TOPK    at least its k largest logits, so the row's k largest are in the lists (a list that overflows is cut to them);
 //     FULL    its logits down to a bound of its own, and the mass exp(x/t - max/t) of the rest. The row's logits above
 //             the largest such bound are then all listed, and the row's whole mass is known.
 //   vs_finish_kernel   finishes each row from its lists, one workgroup per row. A FULL row is finished here if its
 //     top-p cut, min-p cut and draw fall among the logits that are known to be listed (a language model's usual row).
 //   vs_resolve_kernel  takes the rows left open with as many workgroups per row as there are: flat distributions by one
-//     histogram pass and one gather pass over the row, everything else (lists that overflowed, long runs of tied
+//     histogram pass and one gather pass over the row, everything else (FULL lists that overflowed, long runs of tied
 //     values, top-k above the lists' reach, no finite logit) by a radix select over passes. It ends at once when no
-//     row is open. Only here do workgroups wait for one another (a cluster's barrier, bounded in time).
+//     row is open. Only here do workgroups wait for one another (a cluster's barrier, bounded in time); GREEDY rows and
+//     TOPK rows with a finite logit are never left open.
 #include "vs_sample.h"
 
 
@@ -25,7 +26,7 @@ namespace vs {
 constexpr int BATCH_ROWS = 2 * RPL_MAX;  // rows per launch
 constexpr int BATCH_NK = 16;             // listed keys a thread of the finish kernel holds
 constexpr int BSEL = RANK_MAX;           // keys it ranks at most
-constexpr uint32_t L_NONE = ~0u;         // a chunk whose list does not hold what it should
+constexpr uint32_t L_NONE = ~0u;         // a chunk of a FULL row whose list does not hold what it should
 constexpr int SEG_CAP = 256;             // candidates a wave stages at most
 constexpr int RNB = 2048;                // value bins of the resolve kernel
 constexpr int RCAP = 2048;               // keys it gathers
@@ -739,15 +740,78 @@ __global__ __launch_bounds__(SNT, 4) void vs_batch_kernel(SampleArgs A) {
   }
   __syncthreads();
   {
-    int C = 0, off = 0;
-    bool bad = false;
+    int C, off;
+    bool bad;
+    auto total = [&]() {
+      C = off = 0;
+      bad = false;
 #pragma unroll
-    for (int i = 0; i < SNW; ++i) {
-      off += i < wv ? s.segc[i] : 0;
-      C += s.segc[i];
-      bad = bad || s.segc[i] > SEG_CAP;
+      for (int i = 0; i < SNW; ++i) {
+        off += i < wv ? s.segc[i] : 0;
+        C += s.segc[i];
+        bad = bad || s.segc[i] > SEG_CAP;
+      }
+      bad = bad || C > A.kcap;
+    };
+    total();
+    if (__builtin_expect(bad && !full, 0)) {
+      // The bound lets about 1.7 k logits through, runs of tied values all of them. A TOPK list needs its k largest keys:
+      // a bisection for a bound that leaves at least k and no more than fit, on the value, then, where one value is left
+      // and still too many hold it, on the place. It ends at the first bound that does, exactly at k otherwise. Without
+      // it such a row was resolved by a radix select over passes (top_k 200, 20 rows of V = 248320 bf16: 243 us a call
+      // against 83 in launches of vs_sample_kernel).
+      int step = 0, cnt;
+      bool fits;
+      auto count = [&](auto pred) {  // two sets of words in turn: one barrier a step
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < E; ++i) c += (int)__popcll(__ballot(pred(i)));
+        int* x = s.red + (step++ & 1) * SNW;
+        if (ln == 0) x[wv] = c;
+        __syncthreads();
+        cnt = 0;
+        fits = true;
+#pragma unroll
+        for (int i = 0; i < SNW; ++i) {
+          cnt += x[i];
+          fits = fits && x[i] <= SEG_CAP;
+        }
+        fits = fits && cnt <= A.kcap;
+      };
+      auto place = [&](int i) -> int { return ((i / VEC) * SNT + t) * VEC + i % VEC; };  // of v[i], in the order of the ids
+      uint32_t lo = L ? L : ord32(-__FLT_MAX__), hi = ord32(wm) + 1;  // too many from lo up, fewer than k from hi up
+      fits = false;
+      while (!fits && hi - lo > 1) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        const float f = inv_ord32(mid);
+        count([&](int i) { return v[i] >= f; });
+        if (cnt < k) {
+          hi = mid;
+          fits = false;
+        } else {
+          lo = mid;
+        }
+      }
+      const float f = inv_ord32(lo);
+      int pl = -1, ph = SNT * E;  // f's places up to pl are too few, up to ph enough
+      while (!fits && ph - pl > 1) {
+        const int mid = (pl + ph) / 2;
+        count([&](int i) { return v[i] > f || (v[i] == f && place(i) <= mid); });
+        if (cnt < k) {
+          pl = mid;
+          fits = false;
+        } else {
+          ph = mid;
+        }
+      }
+      L = lo;
+      cw = 0;
+#pragma unroll
+      for (int i = 0; i < E; ++i) stage(i, v[i] > f || (v[i] == f && place(i) <= ph));
+      if (ln == 0) s.segc[wv] = cw;
+      __syncthreads();
+      total();
     }
-    bad = bad || C > A.kcap;
     if (!bad)
       for (int j = ln; j < cw; j += WAVE) list[off + j] = key64(__uint_as_float(seg[j].x), (uint32_t)l0 + seg[j].y);
     if (t == 0) {
@@ -777,6 +841,7 @@ struct FinishLds {
   u64 tk[BSEL];       // ranked
   double sum[NRED];
   int nz[SNW];
+  int cnt[2 * SNW];
   int misc[8];
 };
 
@@ -862,6 +927,13 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
     u64* h = (u64*)list_area(A.ws, row);
     for (int i = t; i < (int)(HIST_BYTES / 8); i += SNT) h[i] = 0;
   };
+  if (A.list_k > 0 && n == 0) {  // top-list mode: a row without a finite logit has no entries
+    for (int i = t; i < A.list_k; i += SNT) {
+      A.list_ids[(size_t)grow * A.list_k + i] = -1;
+      A.list_vals[(size_t)grow * A.list_k + i] = -__builtin_inff();
+    }
+    return;
+  }
   // incomplete lists; no finite logit (sampler.py:131-132); a top-k above the lists' reach; quotients that overflow
   if (Lmax == L_NONE || n == 0 ||
       (full && (!(tt > 0.0f) || !is_finite(xs0) || !is_finite(xmin / tt) || (top_k > 0 && top_k < n)))) {
@@ -1002,8 +1074,8 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
     cut = NBIN - 1;
     nsel = wave_sum(cg);
   }
-  if (cut >= (1 << 20) || nsel > BSEL || nsel < 1) {
-    leave_open(full ? ROW_FLAT : ROW_ANY);
+  if (full && (cut >= (1 << 20) || nsel > BSEL || nsel < 1)) {
+    leave_open(ROW_FLAT);
     return;
   }
   VS_TR(A, 10);
@@ -1013,6 +1085,39 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
     if (u >= nu) break;
     if (kk[u] != 0 && bin_of(key_value(kk[u])) > cut) kk[u] = 0;
     mine += kk[u] != 0 ? 1 : 0;
+  }
+  if (__builtin_expect(nsel > BSEL, 0)) {
+    // A TOPK row whose cut bin holds more keys than are ranked (tied values): a bisection on the keys, as in the stream
+    // kernel, until at least keff and at most BSEL are left. There are keff from lo up, fewer from hi up.
+    u64 lo = M, hi = ((u64)ord32(xmax) + 1) << 32;
+    for (int step = 0; nsel > BSEL && hi - lo > 1; ++step) {
+      const u64 mid = lo + (hi - lo) / 2;
+      int c = 0;
+#pragma unroll
+      for (int u = 0; u < BATCH_NK; ++u) {
+        if (u >= nu) break;
+        c += (int)__popcll(__ballot(kk[u] >= mid));
+      }
+      int* x = s.cnt + (step & 1) * SNW;
+      if (ln == 0) x[wv] = c;
+      __syncthreads();
+      c = 0;
+#pragma unroll
+      for (int i = 0; i < SNW; ++i) c += x[i];
+      if (c < keff) {
+        hi = mid;
+      } else {
+        lo = mid;
+        nsel = c;
+      }
+    }
+    mine = 0;
+#pragma unroll
+    for (int u = 0; u < BATCH_NK; ++u) {
+      if (u >= nu) break;
+      if (kk[u] < lo) kk[u] = 0;
+      mine += kk[u] != 0 ? 1 : 0;
+    }
   }
   int at = wave_alloc(mine, &s.misc[4]);
   if (mine) {
@@ -1034,7 +1139,6 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
       A.list_ids[(size_t)grow * A.list_k + i] = i < keff ? (int32_t)key_index(s.tk[i]) : -1;
       A.list_vals[(size_t)grow * A.list_k + i] = i < keff ? key_value(s.tk[i]) : -__builtin_inff();
     }
-    if (t == 0) *flag = ROW_DONE;
   } else if (!full) {
     Smem w = {};
     w.misc = s.misc;
@@ -1179,9 +1283,8 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   __syncthreads();
   const int nitems = s.misc[0];
   if (nitems == 0) return;
-  // workgroups per row: as many as leave a cluster for every row (top lists: one, no waiting); no more rows than
-  // workgroups (batch_plan)
-  const int C = A.list_k > 0 ? 1 : max(1, min(CMAX, (int)gridDim.x / nitems));
+  // workgroups per row: as many as leave a cluster for every row; no more rows than workgroups (batch_plan)
+  const int C = max(1, min(CMAX, (int)gridDim.x / nitems));
   const int nb = gridDim.x, b = blockIdx.x;
   const int l = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;  // a cluster's workgroups on one XCD where they fit
   const int cl = l / C, w = l % C;
@@ -1562,13 +1665,6 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       fin.token = (int32_t)key_index(ld_relaxed64(&o->amkey));
       fin.flags = VS_OUT_NOFINITE;
     }
-    if (A.list_k > 0) {
-      for (int i = t; i < A.list_k; i += SNT) {
-        A.list_ids[(size_t)grow * A.list_k + i] = -1;
-        A.list_vals[(size_t)grow * A.list_k + i] = -__builtin_inff();
-      }
-      return;
-    }
     finish();
     return;
   }
@@ -1653,26 +1749,6 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
     }
     Tk = sk.key;
   }
-  if (A.list_k > 0) {  // top-list mode: the k kept keys, sorted (C == 1)
-    if (t == 0) s.misc[2] = 0;
-    __syncthreads();
-    tiles([&](float x, int id) {
-      u64 key;
-      float xs;
-      if (kept(x, id, key, xs)) {
-        const int p = atomicAdd(&s.misc[2], 1);
-        if (p < RCAP) s.keys[p] = key;
-      }
-    });
-    __syncthreads();
-    u64* srt = (u64*)smem_raw;
-    rank_sort(s.keys, min(s.misc[2], RCAP), srt, k);
-    for (int i = t; i < A.list_k; i += SNT) {
-      A.list_ids[(size_t)grow * A.list_k + i] = i < k ? (int32_t)key_index(srt[i]) : -1;
-      A.list_vals[(size_t)grow * A.list_k + i] = i < k ? key_value(srt[i]) : -__builtin_inff();
-    }
-    return;
-  }
   // sums over the kept set: its size and mass, then (with the mass known) what min-p keeps of it
   auto sums = [&](double S, double pthr, uint32_t* gc, double* gm) -> bool {
     int c = 0;
@@ -1703,7 +1779,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   const double S = ld_relaxed_f64(&o->mass[1]);
   int keep = (int)ld_relaxed(&o->cnt[2]);
   double z = S;
-  uint32_t flags = P.top_k >= 1 && P.top_k <= A.kmax ? 0u : (uint32_t)VS_OUT_COOP;  // the general kernel's route bit
+  uint32_t flags = VS_OUT_COOP;  // the general kernel's route bit
   if (has_tp) {  // sampler.py:145-148
     const double tgt = P.top_p * S;
     const Sel a = select(false, tgt);
@@ -1806,8 +1882,9 @@ int batch_path(SampleArgs a, int dtype, int B, size_t ws_rows, const DevInfo* dv
     void* kargs[] = {&a};
     hipError_t e = hipLaunchKernel(sfn, dim3((unsigned)(a.B * p.G)), dim3(SNT), kargs, stream_lds(p.E * SNT), stream);
     if (e == hipSuccess) e = hipLaunchKernel(ffn, dim3((unsigned)a.B), dim3(SNT), kargs, 0, stream);
-    // one workgroup per CU: all resident, so that a cluster's waits end
-    if (e == hipSuccess) e = hipLaunchKernel(rfn, dim3((unsigned)dv->cus), dim3(SNT), kargs, RESOLVE_LDS, stream);
+    // one workgroup per CU: all resident, so that a cluster's waits end (top lists leave no row open)
+    if (e == hipSuccess && a.list_k == 0)
+      e = hipLaunchKernel(rfn, dim3((unsigned)dv->cus), dim3(SNT), kargs, RESOLVE_LDS, stream);
     if (e != hipSuccess) return hip_fail(e, "vs_sample_batch: launch");
   }
   return VS_OK;

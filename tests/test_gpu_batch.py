@@ -277,3 +277,20 @@ def test_top_lists_of_tied_values(dev, k, dtype):
     for r in range(B):
         ri, rv = DR.topk_sorted(x[r], k)
         assert np.array_equal(ids[r], ri) and np.array_equal(vals[r], rv), (k, r)
+
+
+@pytest.mark.parametrize("B,V,pad,dtype", [(24, 131072, 0, torch.float16), (66, 8192, 0, torch.float32),
+                                           (66, 32771, 1, torch.float32), (48, 163840, 0, torch.bfloat16)])
+def test_top_k_above_the_lists(dev, B, V, pad, dtype):
+    """top_k above 256: gathered by one pass and finished in one workgroup up to 2048, by radix selects above and where
+    too many keys share the cut's bin; rows whose tiles stay in LDS between the passes and (48 rows) rows read again."""
+    rng = np.random.default_rng(V)
+    x = np.concatenate([hard_lists(rng, V, B // 2), (rng.standard_t(3, (B - B // 2, V)) * 3).astype(np.float32)])
+    low = -60000.0 if dtype == torch.float16 else -1e9
+    for r in range(0, B, 4):
+        x[r, rng.random(V) < 0.3] = low  # masked by a large negative value: the values' range says nothing
+    ks = [257, 300, 1000, 2047, 2048, 2049, 5000, 512, 513]
+    ps = [Sampling(top_k=ks[r % 9], top_p=float([1.0, 0.9, 0.3][r % 3]), min_p=float([0.0, 0.0, 0.02, 0.0, 0.3][r % 5]),
+                   temperature=float([1.0, 0.6, 1.8][r % 3])) for r in range(B)]
+    u = (np.floor(rng.random(B) * 4000) + 0.37) / 4000
+    check(dev, x, ps, u, dtype=dtype, pad=pad, label=f"large top-k {B}x{V}", max_excused=1)

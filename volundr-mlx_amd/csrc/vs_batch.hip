@@ -12,8 +12,8 @@
 //   vs_finish_kernel   finishes each row from its lists, one workgroup per row. A FULL row is finished here if its
 //     top-p cut, min-p cut and draw fall among the logits that are known to be listed (a language model's usual row).
 //   vs_resolve_kernel  takes the rows left open with as many workgroups per row as there are: flat distributions by one
-//     histogram pass and one gather pass over the row, everything else (FULL lists that overflowed, long runs of tied
-//     values, top-k above the lists' reach, no finite logit) by a radix select over passes. It ends at once when no
+//     histogram pass and one gather pass over the row, a top-k above the lists' reach likewise, everything else (long
+//     runs of tied values, a top-k of thousands, no finite logit) by a radix select over passes. It ends at once when no
 //     row is open. Only here do workgroups wait for one another (a cluster's barrier, bounded in time); GREEDY rows and
 //     TOPK rows with a finite logit are never left open.
 #include "vs_sample.h"
@@ -38,7 +38,8 @@ constexpr int CMAX = 32;                 // workgroups per open row at most
 // relies on; of a partial all but the word `pad`, by whose tags vs_sample_kernel tells this call's partials from what
 // earlier ones left). The open flags sit in the control blocks' lines, after RowCtl: those of rows [56 k, 56 k + 56) in
 // workspace row k. Nothing here has to be zero when a call starts.
-enum { ROW_DONE = 0, ROW_FLAT = 1, ROW_ANY = 2 };  // open flag: finished, left to the flat or to the general method
+// open flag: finished, left to the flat, the top-k or the general method
+enum { ROW_DONE = 0, ROW_FLAT = 1, ROW_ANY = 2, ROW_TOPK = 3 };
 constexpr size_t OFF_OPEN = 64;
 constexpr int OPEN_PER = 56;
 static_assert(OFF_OPEN >= sizeof(RowCtl) && OFF_OPEN + OPEN_PER <= OFF_PART, "after RowCtl, before the partials");
@@ -55,7 +56,7 @@ __device__ __forceinline__ char* list_area(char* ws, int r) {
 // What the finish kernel leaves of an open row (over its partials), and the row's counters in the resolve kernel.
 struct OpenRow {
   int n;             // finite logits
-  float xmax, xmin;  // the largest and smallest of them
+  float xmax, xmin;  // the largest and smallest of them (ROW_TOPK: a value that the top-k cut hardly lies below)
   uint32_t bar;      // arrivals at the cluster's barriers
   uint32_t gcnt;     // gathered keys
   uint32_t tag;      // the first partial's tag word, left alone
@@ -908,6 +909,10 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
   const float xmax = wave_max(pm), xmin = wave_min(pmn);
   const float tt = P.temperature;
   const float xs0 = xmax / tt;
+  // a top-k cut above the lists' reach: the chunks' bounds lie around the 64 G-th logit; four times as far below the
+  // maximum lies the cut of any top_k that the resolve kernel gathers, unless the row is of an odd shape
+  const uint32_t lmin = wave_min(pl != 0 ? pl : L_NONE);
+  const float xcut = lmin != L_NONE ? fmaxf(xmin, xmax - 4.0f * (xmax - inv_ord32(lmin))) : xmin;
   auto leave_open = [&](int how) {
     __syncthreads();  // the partials and lists are read
     OpenRow* o = (OpenRow*)part_area(A.ws, row);
@@ -915,7 +920,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
       *flag = (uint8_t)how;
       o->n = n;
       o->xmax = xmax;
-      o->xmin = xmin;
+      o->xmin = how == ROW_TOPK ? xcut : xmin;
       o->bar = o->gcnt = 0;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -935,10 +940,10 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
     return;
   }
   // incomplete lists; no finite logit (sampler.py:131-132); a top-k above the lists' reach; quotients that overflow
-  if (Lmax == L_NONE || n == 0 ||
-      (full && (!(tt > 0.0f) || !is_finite(xs0) || !is_finite(xmin / tt) || (top_k > 0 && top_k < n)))) {
-    const bool flat = full && n > 0 && tt > 0.0f && is_finite(xs0) && is_finite(xmin / tt) && !(top_k > 0 && top_k < n);
-    leave_open(flat ? ROW_FLAT : ROW_ANY);
+  const bool cutk = full && top_k > 0 && top_k < n;
+  if (Lmax == L_NONE || n == 0 || cutk || (full && (!(tt > 0.0f) || !is_finite(xs0) || !is_finite(xmin / tt)))) {
+    const bool plain = full && n > 0 && tt > 0.0f && is_finite(xs0) && is_finite(xmin / tt);
+    leave_open(!plain ? ROW_ANY : !cutk ? ROW_FLAT : top_k <= RCAP ? ROW_TOPK : ROW_ANY);
     return;
   }
   // Keys below M are not needed: of a FULL row every key from the largest bound up is listed; a chunk of a TOPK row that
@@ -1327,10 +1332,12 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       for (int e = 0; e < RE; ++e) fn(v[e], l0 + ((e / VEC) * SNT + t) * VEC + e % VEC);
     }
   };
-  // a later pass: from LDS where every tile is resident (each lane reads what it wrote)
+  // a pass that may be a later one: from LDS where every tile is held there (each lane reads what it wrote)
+  bool held = false;
   auto tiles_again = [&](auto fn) {
-    if (!resident) {
+    if (!(resident && held)) {
       tiles(fn);
+      held = true;
       return;
     }
     for (int i = 0; i < m; ++i) {
@@ -1380,6 +1387,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
     };
     if (unit) tiles([&](float x, int) { add_mass(x, x); });
     else tiles([&](float x, int) { add_mass(x, x / tt); });
+    held = true;
     __syncthreads();
     VS_TR(A, 2);
     double* gh = (double*)area;
@@ -1640,7 +1648,194 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       VS_TR_FLUSH(A);
       return;
     }
-    // too many keys in those bins (long runs of tied values): the general method, on cleared histograms
+    // too many keys in those bins (long runs of tied values): the general method
+  } else if (how == ROW_TOPK) {
+    // ---- a top-k cut above the lists' reach: one histogram of counts over value bins, one gather of the bins down to
+    // the one the cut lies in, then workgroup 0 orders the gathered keys by bin and finishes on the k largest. The radix
+    // selects of the general method took nine and more passes for it (top_k 1000, 36 rows of V = 163840 f32: 148 us a
+    // call against 109 in launches of vs_sample_kernel; now 41). ----
+    const int k = P.top_k;
+    const float bsc = xmax > xmin && xmax - xmin < 3.0e38f ? ((float)RNB - 0.5f) / (xmax - xmin) : 0.0f;
+    auto bin_of = [&](float x) -> int { return (int)fminf((xmax - x) * bsc, (float)(RNB - 1)); };
+    uint32_t* hc = (uint32_t*)s.hist;  // [RNB] counts, then their inclusive sums
+    uint32_t* cur = hc + RNB;          // [RNB] the next place of each bin
+    for (int i = t; i < RNB; i += SNT) hc[i] = 0;
+    if (t == 0) {
+      s.misc[2] = 0;
+      s.misc[5] = -1;
+    }
+    __syncthreads();
+    tiles_again([&](float x, int) {
+      if (is_finite(x) & (x >= xmin)) atomicAdd(&hc[bin_of(x)], 1u);
+    });
+    __syncthreads();
+    uint32_t* gh = (uint32_t*)area;
+    if (C > 1) {
+#pragma unroll
+      for (int i = 0; i < RNB / SNT; ++i) {
+        const uint32_t c = hc[t + i * SNT];
+        if (c) atomicAdd(&gh[t + i * SNT], c);
+      }
+      if (!barrier()) {
+        finish();
+        return;
+      }
+    }
+    {  // inclusive sums, in place: thread t owns bins 4 t .. 4 t + 3
+      int c[4], lc = 0, tot;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        c[i] = (int)(C > 1 ? ld_relaxed(&gh[4 * t + i]) : hc[4 * t + i]);
+        lc += c[i];
+      }
+      int cc = block_scan<SNT>(lc, s.red, &tot) - lc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int before = cc;
+        cc += c[i];
+        hc[4 * t + i] = (uint32_t)cc;
+        cur[4 * t + i] = (uint32_t)before;
+        if (cc >= k && before < k) {
+          s.misc[5] = 4 * t + i;
+          s.misc[6] = cc;
+        }
+      }
+    }
+    __syncthreads();
+    const int kb = s.misc[5], ng = kb >= 0 ? s.misc[6] : RCAP + 1;
+    if (ng <= RCAP) {
+      tiles_again([&](float x, int id) {
+        if (is_finite(x) & (x >= xmin) && bin_of(x) <= kb) {
+          const int p = atomicAdd(&s.misc[2], 1);
+          if (p < RCAP) s.keys[p] = key64(x, (uint32_t)id);
+        }
+      });
+      __syncthreads();
+      const int nloc = s.misc[2];
+      if (t == 0) s.misc[3] = (int)atomicAdd(&o->gcnt, (uint32_t)nloc);
+      __syncthreads();
+      const int g0 = s.misc[3];
+      for (int i = t; i < nloc && i < RCAP; i += SNT)
+        if (g0 + i < RCAP) st_dev(&gkeys[g0 + i], s.keys[i]);
+      if (!barrier()) {
+        finish();
+        return;
+      }
+      if (w != 0) return;
+      u64* mem = (u64*)smem_raw;  // [RCAP] the keys, bin by bin
+      u64* srt = mem + RCAP;      // [RCAP] the k largest, in order
+      static_assert(2 * RCAP * 8 <= RESOLVE_LDS && RCAP <= 4 * SNT, "both fit the tile area, four keys per thread");
+      u64 kr[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) kr[i] = t + i * SNT < ng ? ld_dev(&gkeys[t + i * SNT]) : (u64)0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (kr[i]) mem[atomicAdd(&cur[bin_of(key_value(kr[i]))], 1u)] = kr[i];
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (kr[i]) {
+          const int bin = bin_of(key_value(kr[i])), end = (int)hc[bin];
+          int r = bin > 0 ? (int)hc[bin - 1] : 0;
+          for (int j = r; j < end; ++j) r += mem[j] > kr[i] ? 1 : 0;
+          if (r < k) srt[r] = kr[i];
+        }
+      }
+      __syncthreads();
+      // sampler.py:141-156 on srt[0, k): thread t owns positions E t .. E t + E - 1
+      const int E = (k + SNT - 1) / SNT, i0 = E * t;
+      double pr[4], ls = 0.0, S;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        pr[q] = q < E && i0 + q < k ? mass_at(key_value(srt[i0 + q]) / tt - xs0) : 0.0;
+        ls += pr[q];
+      }
+      const double base0 = block_scan<SNT>(ls, s.redd, &S) - ls;
+      const double base = base0 / S;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) pr[q] = pr[q] / S;
+      constexpr int NOWHERE = 1 << 30;
+      int keep = k;
+      uint32_t flags = VS_OUT_COOP;
+      // the first position below `end` whose cumulative mass reaches tgt (NOWHERE: none), its mass and the sum through it
+      // in s.hm[0] and s.hm[1]
+      auto reach = [&](double tgt, int end) -> int {
+        double c = base, hp = 0.0, hc2 = 0.0;
+        int hit = NOWHERE;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (q < E && i0 + q < end) {
+            c += pr[q];
+            if (hit == NOWHERE && c >= tgt) {
+              hit = i0 + q;
+              hp = pr[q];
+              hc2 = c;
+            }
+          }
+        }
+        const int at = block_min<SNT>(hit, s.red);
+        if (at != NOWHERE && at == hit) {
+          s.hm[0] = hp;
+          s.hm[1] = hc2;
+        }
+        __syncthreads();
+        return at;
+      };
+      // the position `at` itself: its mass and the sum through it, likewise
+      auto look = [&](int at) {
+        if (at / E == t) {
+          double c = base, hp = 0.0;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if (q < E && i0 + q <= at) {
+              c += pr[q];
+              hp = pr[q];
+            }
+          }
+          s.hm[0] = hp;
+          s.hm[1] = c;
+        }
+        __syncthreads();
+      };
+      if (has_tp) {  // :145-148
+        const int at = reach(P.top_p, k);
+        if (at != NOWHERE) {
+          keep = at + 1;
+          if (fabs(s.hm[1] - P.top_p) < 1e-6 || fabs(s.hm[1] - s.hm[0] - P.top_p) < 1e-6) flags |= VS_OUT_TOPP_BOUNDARY;
+        }
+      }
+      if (has_mp) {  // :149-152 (the largest key's mass is 1 before the division by S)
+        const double pthr = (1.0 / S) * P.min_p;
+        int hit = NOWHERE;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (hit == NOWHERE && q < E && i0 + q < k && pr[q] < pthr) hit = i0 + q;
+        const int at = block_min<SNT>(hit, s.red);
+        const int cnt = at == NOWHERE ? k : max(at, 1);
+        keep = cnt < keep ? cnt : keep;
+      }
+      __syncthreads();
+      look(keep - 1);
+      const double z = s.hm[1], uz = P.u * z;  // :153-154
+      __syncthreads();
+      int j = reach(uz, keep);
+      if (j == NOWHERE) look(j = keep - 1);  // :155-156
+      const double hp = s.hm[0], hs = s.hm[1], tol = 1e-6 * z;
+      if (fabs(hs - uz) < tol || (j >= 1 && fabs(hs - hp - uz) < tol)) flags |= VS_OUT_DRAW_BOUNDARY;
+      fin.token = (int32_t)key_index(srt[j]);
+      fin.lp = (float)log_ratio(hp, z);
+      fin.keep = keep;
+      fin.flags = flags;
+      finish();
+      return;
+    }
+    // more keys than are gathered (tied values, a row of an odd shape): the general method, once everyone has read the sums
+    if (!barrier()) {
+      finish();
+      return;
+    }
+  }
+  if (how != ROW_ANY) {  // on cleared histograms
     if (w == 0)
       for (int i = t; i < (int)(HIST_BYTES / 8); i += SNT) st_dev((u64*)area + i, (u64)0);
     if (t == 0 && w == 0) st_dev(&o->cnt[2], 0u);
@@ -1653,7 +1848,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   // ---- the general method: exact selections by radix passes on the 64-bit keys ----
   if (n == 0) {  // sampler.py:131-132
     u64 am = 0;
-    tiles([&](float x, int id) {
+    tiles_again([&](float x, int id) {
       if (id >= 0 && id < R.vlim) {
         const u64 k = amkey64(x, (uint32_t)id);
         am = k > am ? k : am;
@@ -1696,7 +1891,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
         s.hk[t] = 0;
       }
       __syncthreads();
-      tiles([&](float x, int id) {
+      tiles_again([&](float x, int id) {
         u64 key;
         float xs;
         if (kept(x, id, key, xs) && prefix_match(key, shift, prefix)) {
@@ -1734,6 +1929,10 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       r.mass_before += q.mass_before;
       prefix = (prefix << 8) | (u64)q.d;
       __syncthreads();
+      if (by_count && (double)(r.cnt_before + q.cnt) == target) {  // the digit is kept whole: its lowest key bounds the cut
+        r.key = prefix << shift;
+        return r;
+      }
       if (q.cnt <= 1 || shift == 0) {
         r.key = q.mk;
         r.mass = q.mass;
@@ -1753,7 +1952,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   auto sums = [&](double S, double pthr, uint32_t* gc, double* gm) -> bool {
     int c = 0;
     double f = 0.0;
-    tiles([&](float x, int id) {
+    tiles_again([&](float x, int id) {
       u64 key;
       float xs;
       if (kept(x, id, key, xs)) {

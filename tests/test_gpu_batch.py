@@ -294,3 +294,21 @@ def test_top_k_above_the_lists(dev, B, V, pad, dtype):
                    temperature=float([1.0, 0.6, 1.8][r % 3])) for r in range(B)]
     u = (np.floor(rng.random(B) * 4000) + 0.37) / 4000
     check(dev, x, ps, u, dtype=dtype, pad=pad, label=f"large top-k {B}x{V}", max_excused=1)
+
+
+@pytest.mark.parametrize("kind", ["flat", "min_p", "tied", "top_k"])
+def test_open_rows_repeat_bit_for_bit(dev, kind):
+    """Rows that several workgroups finish together add their masses up in an order of no kind: the results must not
+    depend on it."""
+    rng = np.random.default_rng(21)
+    B, V = 66, 40000
+    x = (rng.standard_normal((B, V)) * (0.1 if kind != "top_k" else 2.0)).astype(np.float32)
+    if kind == "tied":
+        x = np.round(x * 20) / 20
+    kw = dict(flat=dict(top_p=0.9), min_p=dict(min_p=0.7), tied=dict(top_p=0.9, min_p=0.7), top_k=dict(top_k=6000))[kind]
+    rows = ops.pack_rows([Sampling(temperature=0.9, **kw)] * B, rng.random(B), V).to(dev)
+    xt = torch.from_numpy(x).to(dev)
+    print(f"[repeat] {kind}", flush=True)
+    first = ops.sample_rows(xt, rows).block.clone()
+    for _ in range(12):
+        assert torch.equal(ops.sample_rows(xt, rows).block, first)

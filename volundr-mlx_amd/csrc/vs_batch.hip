@@ -61,14 +61,15 @@ struct OpenRow {
   uint32_t gcnt;     // gathered keys
   uint32_t tag;      // the first partial's tag word, left alone
   uint32_t cnt[4];   // sums over the cluster: counts
-  double mass[4];    // and masses
+  int shift;         // masses are summed in fixed point at 2^shift: the whole row's stay below 2^63
+  u64 fix[3];        // and masses
   u64 amkey;
 };
 static_assert(offsetof(OpenRow, tag) == offsetof(Part, pad) && sizeof(OpenRow) <= sizeof(Part), "the tag words stay");
 // An open row's list area: the mass histogram of the flat method (or the ring of radix histograms), then the keys.
 struct RadixSlot {
   uint32_t cnt[NBIN];
-  double mass[NBIN];
+  u64 fix[NBIN];
   u64 mk[NBIN];
 };
 constexpr size_t HIST_BYTES = RNB * 8;
@@ -820,7 +821,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_batch_kernel(SampleArgs A) {
 #pragma unroll
       for (int i = 0; i < SNW; ++i) r += s.sum[i];
       part->nfin = (uint32_t)nf;
-      part->kc = (uint32_t)(bad ? 0 : C);
+      part->kc = (uint32_t)C;
       part->heads[1] = bad ? L_NONE : L;  // (the tag word `pad` is vs_sample_kernel's alone)
       part->heads[0] = ((u64)__float_as_uint(wm) << 32) | __float_as_uint(mn);
       part->se = r;
@@ -914,6 +915,10 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
   const uint32_t lmin = wave_min(pl != 0 ? pl : L_NONE);
   const float xcut = lmin != L_NONE ? fmaxf(xmin, xmax - 4.0f * (xmax - inv_ord32(lmin))) : xmin;
   auto leave_open = [&](int how) {
+    // 63 bits for the row's mass: at most each chunk's unlisted mass and 1 for every listed logit, times the chunk's maximum
+    const double most = wave_sum(pn ? (pp.se + (double)cg) * (double)expf(pm / tt - xs0) : 0.0) * 1.001;
+    const int fits = most >= 1.0 && most < 1e9 ? 62 - ilogb(most) : A.fix_shift;
+    const int shift = fits > A.fix_shift ? fits : A.fix_shift;
     __syncthreads();  // the partials and lists are read
     OpenRow* o = (OpenRow*)part_area(A.ws, row);
     if (t == 0) {
@@ -925,9 +930,10 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         o->cnt[i] = 0;
-        o->mass[i] = 0.0;
+        if (i < 3) o->fix[i] = 0;
       }
       o->amkey = 0;
+      o->shift = shift;
     }
     u64* h = (u64*)list_area(A.ws, row);
     for (int i = t; i < (int)(HIST_BYTES / 8); i += SNT) h[i] = 0;
@@ -1190,15 +1196,16 @@ constexpr int RKEEP = 3;                        // tiles whose edited logits sta
 constexpr size_t RESOLVE_LDS = (size_t)RKEEP * RTILE * 4;  // the tiles: their edit words, then their logits
 
 // exp(x/t - max/t), sampler.py:141-142 (below e^-150, a float zero, the argument would only overflow in exp_nonpos)
-__device__ __forceinline__ double mass_at(float d) { return (double)exp_nonpos(fmaxf(d, -150.0f)); }
+__device__ __forceinline__ float mass_at(float d) { return exp_nonpos(fmaxf(d, -150.0f)); }
 
 struct ResolveLds {
-  double hist[RNB];   // flat method: masses by value bin, then their inclusive sums
+  u64 hist[RNB];      // flat method: masses by value bin, then their inclusive sums
   u64 keys[RCAP];     // gathered keys
   uint32_t hc[NBIN];  // radix: counts, masses, largest keys by digit
-  double hm[NBIN];
+  u64 hm[NBIN];
   u64 hk[NBIN];
   double redd[NRED];
+  double at[2];       // a position's mass and the sum through it
   u64 red64[NRED];
   int red[NRED];
   int misc[16];
@@ -1210,14 +1217,13 @@ struct ResolveLds {
 struct Digit {
   int d;
   uint32_t cnt_before, cnt;
-  double mass_before, mass;
+  u64 mass_before, mass;  // in fixed point
   u64 mk;
 };
-__device__ __forceinline__ Digit find_digit(const uint32_t* hc, const double* hm, const u64* hk, bool by_count,
-                                            double target) {
+__device__ __forceinline__ Digit find_digit(const uint32_t* hc, const u64* hm, const u64* hk, bool by_count, u64 target) {
   const int L = lane_id();
   uint32_t c[4], lc = 0;
-  double f[4], lf = 0.0;
+  u64 f[4], lf = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int d = NBIN - 1 - (4 * L + i);
@@ -1227,17 +1233,17 @@ __device__ __forceinline__ Digit find_digit(const uint32_t* hc, const double* hm
     lf += f[i];
   }
   uint32_t cc = wave_scan(lc) - lc;
-  double cf = wave_scan(lf) - lf;
+  u64 cf = wave_scan(lf) - lf;
   int hit = -1, last = -1;
   uint32_t cb = 0, lcb = 0;
-  double fb = 0.0, lfb = 0.0;
+  u64 fb = 0, lfb = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if (c[i] > 0) {
       last = i;
       lcb = cc;
       lfb = cf;
-      if (hit < 0 && (by_count ? (double)(cc + c[i]) : cf + f[i]) >= target) {
+      if (hit < 0 && (by_count ? (u64)(cc + c[i]) : cf + f[i]) >= target) {
         hit = i;
         cb = cc;
         fb = cf;
@@ -1370,6 +1376,12 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   const bool filt = n > 4096;
   const float thr = filt ? xs0 - 40.0f : -__builtin_inff();  // sampler.py:137-139
   const bool has_tp = P.top_p < 1.0, has_mp = P.min_p > 0.0;
+  // Masses are summed in fixed point: the sums do not depend on the order of the additions, so a call's cuts, draws and
+  // logprobs are the same every time. A mass is rounded by 2^-63 of the row's at most, no more than float64 sums of as
+  // many terms lose. (64 near-flat rows of V = 163840 f32 take 65.2 us a call, 63.6 with float64 sums.)
+  const float fsc = __builtin_amdgcn_ldexpf(1.0f, o->shift), fsh = __builtin_amdgcn_ldexpf(1.0f, o->shift - 32);
+  const double inv_scale = 1.0 / (double)fsc;
+  auto fix_of = [&](float e) -> u64 { return fixed_mass(e, fsh, fsc); };
 
   VS_TR(A, 1);
   if (how == ROW_FLAT) {
@@ -1378,24 +1390,24 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
     const float xl = filt ? fmaxf(xmin, xmax - 40.0f * tt * 1.00001f - 1e-30f) : xmin;
     const float bsc = xmax > xl && xmax - xl < 3.0e38f ? ((float)RNB - 0.5f) / (xmax - xl) : 0.0f;
     auto bin_of = [&](float x) -> int { return (int)fminf((xmax - x) * bsc, (float)(RNB - 1)); };
-    for (int i = t; i < RNB; i += SNT) s.hist[i] = 0.0;
+    for (int i = t; i < RNB; i += SNT) s.hist[i] = 0;
     if (t == 0) s.misc[2] = 0;
     __syncthreads();
     const bool unit = tt == 1.0f;  // x / 1 == x: no division
     auto add_mass = [&](float x, float xs) {
-      if (is_finite(x) & (xs >= thr)) unsafeAtomicAdd(&s.hist[bin_of(x)], mass_at(xs - xs0));
+      if (is_finite(x) & (xs >= thr)) atomicAdd(&s.hist[bin_of(x)], fix_of(mass_at(xs - xs0)));
     };
     if (unit) tiles([&](float x, int) { add_mass(x, x); });
     else tiles([&](float x, int) { add_mass(x, x / tt); });
     held = true;
     __syncthreads();
     VS_TR(A, 2);
-    double* gh = (double*)area;
+    u64* gh = (u64*)area;
     if (C > 1) {
 #pragma unroll
       for (int i = 0; i < RNB / SNT; ++i) {
-        const double f = s.hist[t + i * SNT];
-        if (f != 0.0) unsafeAtomicAdd(&gh[t + i * SNT], f);
+        const u64 f = s.hist[t + i * SNT];
+        if (f != 0) atomicAdd(&gh[t + i * SNT], f);
       }
       if (!barrier()) {
         finish();
@@ -1405,15 +1417,15 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
     VS_TR(A, 3);
     // inclusive sums, in place: thread t owns bins 4 t .. 4 t + 3
     static_assert(RNB == 4 * SNT, "four bins per thread");
-    double c4[4], cprev, S;
+    u64 c4[4], cprev, Sfix;
     {
-      double f[4], lf = 0.0;
+      u64 f[4], lf = 0;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        f[i] = C > 1 ? ld_relaxed_f64(&gh[4 * t + i]) : s.hist[4 * t + i];
+        f[i] = C > 1 ? ld_relaxed64(&gh[4 * t + i]) : s.hist[4 * t + i];
         lf += f[i];
       }
-      double c = block_scan<SNT>(lf, s.redd, &S) - lf;
+      u64 c = block_scan<SNT>(lf, s.red64, &Sfix) - lf;
       cprev = c;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1424,20 +1436,20 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
     }
     if (t == 0) s.misc[5] = s.misc[6] = s.misc[7] = RNB - 1;
     __syncthreads();
-    S = s.hist[RNB - 1];
-    // the first bin whose inclusive sum reaches target, into misc[at] by its owner (target <= S)
+    const double S = (double)Sfix * inv_scale;
+    // the first bin whose inclusive sum reaches target (fixed point), into misc[at] by its owner
     auto find = [&](double target, int at) {
-      const double tg = fmin(fmax(target, 5e-324), S);
-      double prev = cprev;
+      u64 tg = ceil_u64(target), prev = cprev;
+      tg = tg < 1 ? 1 : (tg > Sfix ? Sfix : tg);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         if (c4[i] >= tg && prev < tg) s.misc[at] = 4 * t + i;
         prev = c4[i];
       }
     };
-    auto before = [&](int bin) -> double { return bin > 0 ? s.hist[bin - 1] : 0.0; };
-    const double tgt_p = P.top_p * S;
-    double zlo = S, zhi = S;
+    auto before = [&](int bin) -> u64 { return bin > 0 ? s.hist[bin - 1] : 0; };
+    const double tgt_p = P.top_p * (double)Sfix;
+    u64 zlo = Sfix, zhi = Sfix;
     int T = -1;
     if (has_tp) {
       find(tgt_p, 5);
@@ -1451,27 +1463,27 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       // the kept prefix ends between the values log(min_p) -+ 1e-4 below the maximum (in units of the temperature)
       const float lg = logf((float)P.min_p), sl = 1e-4f + 1e-5f * fabsf(xs0);
       const float xa = xmax + tt * fminf(lg + sl, 0.0f), xb = xmax + tt * fminf(lg - sl, 0.0f);
-      zlo = fmin(zlo, before(bin_of(fmaxf(xa, xl))));
-      zhi = fmin(zhi, s.hist[bin_of(fmaxf(xb, xl))]);
-      zlo = fmin(zlo, zhi);
+      zlo = min(zlo, before(bin_of(fmaxf(xa, xl))));
+      zhi = min(zhi, s.hist[bin_of(fmaxf(xb, xl))]);
+      zlo = min(zlo, zhi);
     }
-    find(P.u * zlo * (1.0 - 1e-9), 6);
-    find(P.u * zhi * (1.0 + 1e-9), 7);
+    find(P.u * (double)zlo * (1.0 - 1e-9), 6);
+    find(P.u * (double)zhi * (1.0 + 1e-9), 7);
     __syncthreads();
     const int D0 = s.misc[6], D1 = s.misc[7];
     VS_TR(A, 4);
     int cT = 0, cM = 0, kc = 0;
-    double mM = 0.0;
+    u64 fM = 0;
     auto take = [&](float x, float xs, int id) {
       if (is_finite(x) & (xs >= thr)) {
         const int bin = bin_of(x);
         ++kc;
         cT += bin < T ? 1 : 0;
         if (has_mp) {
-          const double pr = mass_at(xs - xs0);
-          if (!(pr / S < pthr)) {
+          const float e = mass_at(xs - xs0);
+          if (!((double)e / S < pthr)) {
             ++cM;
-            mM += pr;
+            fM += fix_of(e);
           }
         }
         if ((bin == T) | ((bin >= D0) & (bin <= D1))) {
@@ -1486,14 +1498,14 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
     cT = block_sum<SNT>(cT, s.red);
     kc = block_sum<SNT>(kc, s.red);
     cM = has_mp ? block_sum<SNT>(cM, s.red) : 0;
-    mM = has_mp ? block_sum<SNT>(mM, s.redd) : 0.0;
+    fM = has_mp ? block_sum<SNT>(fM, s.red64) : 0;
     const int nloc = s.misc[2];
     if (t == 0) {
       if (cT) atomicAdd(&o->cnt[0], (uint32_t)cT);
       if (kc) atomicAdd(&o->cnt[2], (uint32_t)kc);
       if (has_mp) {
         atomicAdd(&o->cnt[1], (uint32_t)cM);
-        unsafeAtomicAdd(&o->mass[0], mM);
+        atomicAdd(&o->fix[0], fM);
       }
       s.misc[3] = (int)atomicAdd(&o->gcnt, (uint32_t)nloc);
     }
@@ -1514,7 +1526,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       }
       const int cnt_t = (int)ld_relaxed(&o->cnt[0]), cnt_m = (int)ld_relaxed(&o->cnt[1]);
       const int total = (int)ld_relaxed(&o->cnt[2]);
-      const double mass_m = ld_relaxed_f64(&o->mass[0]);
+      const u64 fix_m = ld_relaxed64(&o->fix[0]);
       u64* mem = (u64*)smem_raw;  // [RCAP] members
       static_assert(RCAP * 8 <= RESOLVE_LDS, "the members fit the tile area");
       u64 kr[RCAP / SNT];
@@ -1522,23 +1534,23 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       for (int i = 0; i < RCAP / SNT; ++i) kr[i] = t + i * SNT < ng ? ld_dev(&gkeys[t + i * SNT]) : (u64)0;
       struct Pick {
         u64 key;
-        int rank;             // members above it
-        double below, mass;   // the mass above it, its own
+        int rank;         // members above it
+        u64 below, mass;  // the mass above it, its own
       };
-      auto mass_of = [&](u64 key) -> double { return mass_at(key_value(key) / tt - xs0); };
+      auto mass_of = [&](u64 key) -> u64 { return fix_of(mass_at(key_value(key) / tt - xs0)); };
       auto clear = [&]() {
         __syncthreads();
         if (t < NBIN) {
           s.hc[t] = 0;
-          s.hm[t] = 0.0;
+          s.hm[t] = 0;
           s.hk[t] = 0;
         }
         __syncthreads();
       };
       // The first member of `bin`, in descending order, at which the bin's mass reaches tgt (the last if none): by
       // 256 parts of the bin, then among the few members of the part.
-      auto pick = [&](int bin, double tgt) -> Pick {
-        Pick r = {0, 0, 0.0, 0.0};
+      auto pick = [&](int bin, u64 tgt) -> Pick {
+        Pick r = {0, 0, 0, 0};
         auto part_of = [&](u64 key) -> int {  // 255 .. 0 as the value falls, -1: another bin
           const float p = fminf((xmax - key_value(key)) * bsc, (float)(RNB - 1)), f = p - (float)(int)p;
           return key != 0 && (int)p == bin ? NBIN - 1 - (int)(f * 255.99f) : -1;
@@ -1550,7 +1562,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
           const int d = part_of(kr[i]);
           if (d >= 0) {
             atomicAdd(&s.hc[d], 1u);
-            unsafeAtomicAdd(&s.hm[d], mass_of(kr[i]));
+            atomicAdd(&s.hm[d], mass_of(kr[i]));
           }
         }
         __syncthreads();
@@ -1566,14 +1578,14 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
         if (nm <= WAVE) {  // every wave: lane L holds member L and sums the members above it
           const int L = lane_id();
           const u64 ki = L < nm ? mem[L] : (u64)0;
-          const double me = ki ? mass_of(ki) : 0.0;
+          const u64 me = ki ? mass_of(ki) : 0;
           int rk = 0;
-          double ab = 0.0;
+          u64 ab = 0;
           for (int j = 0; j < nm; ++j) {
             const bool gt = lane_bcast(ki, j) > ki;
-            const double mj = lane_bcast(me, j);
+            const u64 mj = lane_bcast(me, j);
             rk += gt ? 1 : 0;
-            ab += gt ? mj : 0.0;
+            ab += gt ? mj : (u64)0;
           }
           const int hit = wave_min(ki && r.below + ab + me >= tgt ? rk : nm - 1);
           const int ln = __ffsll((long long)__ballot(ki != 0 && rk == hit)) - 1;
@@ -1591,12 +1603,12 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
             if (prefix_match(key, shift, prefix)) {
               const int d = (int)((key >> shift) & 0xFF);
               atomicAdd(&s.hc[d], 1u);
-              unsafeAtomicAdd(&s.hm[d], mass_of(key));
+              atomicAdd(&s.hm[d], mass_of(key));
               atomicMax(&s.hk[d], key);
             }
           }
           __syncthreads();
-          const Digit q = find_digit(s.hc, s.hm, s.hk, false, tgt - r.below);
+          const Digit q = find_digit(s.hc, s.hm, s.hk, false, tgt > r.below ? tgt - r.below : 0);
           r.rank += (int)q.cnt_before;
           r.below += q.mass_before;
           prefix = (prefix << 8) | (u64)q.d;
@@ -1609,7 +1621,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       };
       uint32_t flags = VS_OUT_COOP | (has_mp ? 0u : (uint32_t)VS_OUT_GATHER);
       int keep = total;
-      double z = S;
+      u64 zfix = Sfix;
       bool good = true;
 #pragma nounroll
       for (int draw = has_tp ? 0 : 1; draw < 2; ++draw) {  // the top-p cut, then the draw: one instance of the pick
@@ -1620,24 +1632,25 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
             const int km = cnt_m > 1 ? cnt_m : 1;
             if (km < keep) {
               keep = km;
-              z = cnt_m >= 1 ? mass_m : 1.0;
+              zfix = cnt_m >= 1 ? fix_m : (u64)fsc;
             }
           }
-          tgt = P.u * z;  // :153-156
+          tgt = P.u * (double)zfix;  // :153-156
           bin = D0;
-          while (bin < D1 && s.hist[bin] < tgt) ++bin;
+          while (bin < D1 && s.hist[bin] < ceil_u64(tgt)) ++bin;
         }
-        const Pick pk = pick(bin, tgt - before(bin));
+        const u64 bb = before(bin), tg = ceil_u64(tgt);
+        const Pick pk = pick(bin, tg > bb ? tg - bb : 0);
         good = good && pk.key != 0;
-        const double bef = before(bin) + pk.below, tol = 1e-6 * (draw ? z : S);
-        if (fabs(bef - tgt) < tol || fabs(bef + pk.mass - tgt) < tol)
+        const double bef = (double)(bb + pk.below), tol = 1e-6 * (double)(draw ? zfix : Sfix);
+        if (fabs(bef - tgt) < tol || fabs(bef + (double)pk.mass - tgt) < tol)
           flags |= draw ? VS_OUT_DRAW_BOUNDARY : VS_OUT_TOPP_BOUNDARY;
         if (!draw) {  // :145-148
           keep = cnt_t + pk.rank + 1;
-          z = bef + pk.mass;
+          zfix = bb + pk.below + pk.mass;
         } else if (good) {
           fin.token = (int32_t)key_index(pk.key);
-          fin.lp = (float)((double)(key_value(pk.key) / tt - xs0) - log_ge1(z));
+          fin.lp = (float)((double)(key_value(pk.key) / tt - xs0) - log_ge1((double)zfix * inv_scale));
           fin.keep = keep;
           fin.flags = flags;
         }
@@ -1747,7 +1760,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       double pr[4], ls = 0.0, S;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        pr[q] = q < E && i0 + q < k ? mass_at(key_value(srt[i0 + q]) / tt - xs0) : 0.0;
+        pr[q] = q < E && i0 + q < k ? (double)mass_at(key_value(srt[i0 + q]) / tt - xs0) : 0.0;
         ls += pr[q];
       }
       const double base0 = block_scan<SNT>(ls, s.redd, &S) - ls;
@@ -1758,7 +1771,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       int keep = k;
       uint32_t flags = VS_OUT_COOP;
       // the first position below `end` whose cumulative mass reaches tgt (NOWHERE: none), its mass and the sum through it
-      // in s.hm[0] and s.hm[1]
+      // in s.at[0] and s.at[1]
       auto reach = [&](double tgt, int end) -> int {
         double c = base, hp = 0.0, hc2 = 0.0;
         int hit = NOWHERE;
@@ -1775,8 +1788,8 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
         }
         const int at = block_min<SNT>(hit, s.red);
         if (at != NOWHERE && at == hit) {
-          s.hm[0] = hp;
-          s.hm[1] = hc2;
+          s.at[0] = hp;
+          s.at[1] = hc2;
         }
         __syncthreads();
         return at;
@@ -1792,8 +1805,8 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
               hp = pr[q];
             }
           }
-          s.hm[0] = hp;
-          s.hm[1] = c;
+          s.at[0] = hp;
+          s.at[1] = c;
         }
         __syncthreads();
       };
@@ -1801,7 +1814,8 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
         const int at = reach(P.top_p, k);
         if (at != NOWHERE) {
           keep = at + 1;
-          if (fabs(s.hm[1] - P.top_p) < 1e-6 || fabs(s.hm[1] - s.hm[0] - P.top_p) < 1e-6) flags |= VS_OUT_TOPP_BOUNDARY;
+          if (fabs(s.at[1] - P.top_p) < 1e-6 || fabs(s.at[1] - s.at[0] - P.top_p) < 1e-6)
+            flags |= VS_OUT_TOPP_BOUNDARY;
         }
       }
       if (has_mp) {  // :149-152 (the largest key's mass is 1 before the division by S)
@@ -1816,11 +1830,11 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       }
       __syncthreads();
       look(keep - 1);
-      const double z = s.hm[1], uz = P.u * z;  // :153-154
+      const double z = s.at[1], uz = P.u * z;  // :153-154
       __syncthreads();
       int j = reach(uz, keep);
       if (j == NOWHERE) look(j = keep - 1);  // :155-156
-      const double hp = s.hm[0], hs = s.hm[1], tol = 1e-6 * z;
+      const double hp = s.at[0], hs = s.at[1], tol = 1e-6 * z;
       if (fabs(hs - uz) < tol || (j >= 1 && fabs(hs - hp - uz) < tol)) flags |= VS_OUT_DRAW_BOUNDARY;
       fin.token = (int32_t)key_index(srt[j]);
       fin.lp = (float)log_ratio(hp, z);
@@ -1838,7 +1852,10 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   if (how != ROW_ANY) {  // on cleared histograms
     if (w == 0)
       for (int i = t; i < (int)(HIST_BYTES / 8); i += SNT) st_dev((u64*)area + i, (u64)0);
-    if (t == 0 && w == 0) st_dev(&o->cnt[2], 0u);
+    if (t == 0 && w == 0) {  // (the flat method's sums)
+      st_dev(&o->cnt[2], 0u);
+      st_dev(&o->fix[0], (u64)0);
+    }
     if (!barrier()) {
       finish();
       return;
@@ -1879,15 +1896,15 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   struct Sel {
     u64 key;
     uint32_t cnt_before;
-    double mass_before, mass;
+    u64 mass_before, mass;
   };
-  auto select = [&](bool by_count, double target) -> Sel {
-    Sel r = {0, 0, 0.0, 0.0};
+  auto select = [&](bool by_count, u64 target) -> Sel {
+    Sel r = {0, 0, 0, 0};
     u64 prefix = 0;
     for (int shift = 56;; shift -= 8) {
       if (t < NBIN) {
         s.hc[t] = 0;
-        s.hm[t] = 0.0;
+        s.hm[t] = 0;
         s.hk[t] = 0;
       }
       __syncthreads();
@@ -1897,7 +1914,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
         if (kept(x, id, key, xs) && prefix_match(key, shift, prefix)) {
           const int d = (int)((key >> shift) & 0xFF);
           atomicAdd(&s.hc[d], 1u);
-          if (!by_count) unsafeAtomicAdd(&s.hm[d], mass_at(xs - xs0));
+          if (!by_count) atomicAdd(&s.hm[d], fix_of(mass_at(xs - xs0)));
           atomicMax(&s.hk[d], key);
         }
       });
@@ -1905,31 +1922,31 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       RadixSlot* h = ring + round % RRING;
       if (t < NBIN && s.hc[t]) {
         atomicAdd(&h->cnt[t], s.hc[t]);
-        if (!by_count) unsafeAtomicAdd(&h->mass[t], s.hm[t]);
+        if (!by_count) atomicAdd(&h->fix[t], s.hm[t]);
         atomicMax(&h->mk[t], s.hk[t]);
       }
       // the next round's slot was last read after the barrier before the last one, which every workgroup has left
       if (w == 0 && round >= RRING - 1 && t < NBIN) {
         RadixSlot* z = ring + (round + 1) % RRING;
         st_dev(&z->cnt[t], 0u);
-        st_dev(&z->mass[t], 0.0);
+        st_dev(&z->fix[t], (u64)0);
         st_dev(&z->mk[t], (u64)0);
       }
       ++round;
       if (!barrier()) return r;
       if (t < NBIN) {
         s.hc[t] = ld_relaxed(&h->cnt[t]);
-        s.hm[t] = ld_relaxed_f64(&h->mass[t]);
+        s.hm[t] = ld_relaxed64(&h->fix[t]);
         s.hk[t] = ld_relaxed64(&h->mk[t]);
       }
       __syncthreads();
-      const Digit q = find_digit(s.hc, s.hm, s.hk, by_count,
-                                 by_count ? target - (double)r.cnt_before : target - r.mass_before);
+      const u64 above = by_count ? (u64)r.cnt_before : r.mass_before;
+      const Digit q = find_digit(s.hc, s.hm, s.hk, by_count, target > above ? target - above : 0);
       r.cnt_before += q.cnt_before;
       r.mass_before += q.mass_before;
       prefix = (prefix << 8) | (u64)q.d;
       __syncthreads();
-      if (by_count && (double)(r.cnt_before + q.cnt) == target) {  // the digit is kept whole: its lowest key bounds the cut
+      if (by_count && (u64)(r.cnt_before + q.cnt) == target) {  // the digit is kept whole: its lowest key bounds the cut
         r.key = prefix << shift;
         return r;
       }
@@ -1941,74 +1958,76 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
     }
   };
   if (cutk) {
-    const Sel sk = select(true, (double)k);
+    const Sel sk = select(true, (u64)k);
     if (!ok) {
       finish();
       return;
     }
     Tk = sk.key;
   }
-  // sums over the kept set: its size and mass, then (with the mass known) what min-p keeps of it
-  auto sums = [&](double S, double pthr, uint32_t* gc, double* gm) -> bool {
+  // sums over the kept set: its size and mass, or (with the mass known) those of what min-p keeps of it
+  auto sums = [&](double S, double pthr, int at) -> bool {
     int c = 0;
-    double f = 0.0;
+    u64 f = 0;
     tiles_again([&](float x, int id) {
       u64 key;
       float xs;
       if (kept(x, id, key, xs)) {
-        const double pr = mass_at(xs - xs0);
-        if (S == 0.0 || !(pr / S < pthr)) {
+        const float e = mass_at(xs - xs0);
+        if (S == 0.0 || !((double)e / S < pthr)) {
           ++c;
-          f += pr;
+          f += fix_of(e);
         }
       }
     });
     c = block_sum<SNT>(c, s.red);
-    f = block_sum<SNT>(f, s.redd);
+    f = block_sum<SNT>(f, s.red64);
     if (t == 0) {
-      atomicAdd(gc, (uint32_t)c);
-      unsafeAtomicAdd(gm, f);
+      atomicAdd(&o->cnt[at + 1], (uint32_t)c);
+      atomicAdd(&o->fix[at], f);
     }
     return barrier();
   };
-  if (!sums(0.0, 0.0, &o->cnt[2], &o->mass[1])) {
+  if (!sums(0.0, 0.0, 1)) {
     finish();
     return;
   }
-  const double S = ld_relaxed_f64(&o->mass[1]);
+  const u64 Sfix = ld_relaxed64(&o->fix[1]);
   int keep = (int)ld_relaxed(&o->cnt[2]);
-  double z = S;
+  u64 zfix = Sfix;
   uint32_t flags = VS_OUT_COOP;  // the general kernel's route bit
   if (has_tp) {  // sampler.py:145-148
-    const double tgt = P.top_p * S;
-    const Sel a = select(false, tgt);
+    const double tgt = P.top_p * (double)Sfix;
+    const Sel a = select(false, ceil_u64(tgt));
     if (!ok) {
       finish();
       return;
     }
     keep = (int)a.cnt_before + 1;
-    z = a.mass_before + a.mass;
-    const double tol = 1e-6 * S;
-    if (fabs(a.mass_before - tgt) < tol || fabs(z - tgt) < tol) flags |= VS_OUT_TOPP_BOUNDARY;
+    zfix = a.mass_before + a.mass;
+    const double tol = 1e-6 * (double)Sfix;
+    if (fabs((double)a.mass_before - tgt) < tol || fabs((double)zfix - tgt) < tol) flags |= VS_OUT_TOPP_BOUNDARY;
   }
   if (has_mp) {  // :149-152
-    if (!sums(S, (1.0 / S) * P.min_p, &o->cnt[3], &o->mass[2])) {
+    const double S = (double)Sfix * inv_scale;
+    if (!sums(S, (1.0 / S) * P.min_p, 2)) {
       finish();
       return;
     }
     const int cm = (int)ld_relaxed(&o->cnt[3]), km = cm > 1 ? cm : 1;
     if (km < keep) {
       keep = km;
-      z = cm >= 1 ? ld_relaxed_f64(&o->mass[2]) : 1.0;
+      zfix = cm >= 1 ? ld_relaxed64(&o->fix[2]) : (u64)fsc;
     }
   }
-  const double uz = P.u * z;  // :153-156
-  const Sel d = select(false, uz);
+  const double uz = P.u * (double)zfix;  // :153-156
+  const Sel d = select(false, ceil_u64(uz));
   if (ok && d.key != 0) {
-    const double tol = 1e-6 * z;
-    if (fabs(d.mass_before - uz) < tol || fabs(d.mass_before + d.mass - uz) < tol) flags |= VS_OUT_DRAW_BOUNDARY;
+    const double tol = 1e-6 * (double)zfix;
+    if (fabs((double)d.mass_before - uz) < tol || fabs((double)(d.mass_before + d.mass) - uz) < tol)
+      flags |= VS_OUT_DRAW_BOUNDARY;
     fin.token = (int32_t)key_index(d.key);
-    fin.lp = (float)((double)(key_value(d.key) / tt - xs0) - log_ge1(z));
+    fin.lp = (float)((double)(key_value(d.key) / tt - xs0) - log_ge1((double)zfix * inv_scale));
     fin.keep = keep;
     fin.flags = flags;
   }

@@ -259,7 +259,7 @@ def test_top_k_above_what_a_bound_lists(dev, B, V, pad, dtype):
     """top_k up to 256 where the chunks' bounds let more candidates through than a list holds."""
     rng = np.random.default_rng(B)
     x = hard_lists(rng, V, B)
-    ps = [Sampling(top_k=int([256, 100, 200, 160, 128, 255, 64][r % 7]), top_p=float([1.0, 0.9][r % 2]), temperature=1.3)
+    ps = [Sampling(top_k=int([256, 100, 200, 127, 129, 160, 128, 255, 64][r % 9]), top_p=float([1.0, 0.9][r % 2]), temperature=1.3)
           for r in range(B)]
     u = (np.floor(rng.random(B) * 4000) + 0.37) / 4000  # equal masses: draws off the multiples of 1 / n
     check(dev, x, ps, u, dtype=dtype, pad=pad, label=f"top-k lists {B}x{V}", max_excused=1)

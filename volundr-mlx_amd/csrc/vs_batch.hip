@@ -911,10 +911,11 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
   const float xmax = wave_max(pm), xmin = wave_min(pmn);
   const float tt = P.temperature;
   const float xs0 = xmax / tt;
-  // a top-k cut above the lists' reach: the chunks' bounds lie around the 64 G-th logit; four times as far below the
-  // maximum lies the cut of any top_k that the resolve kernel gathers, unless the row is of an odd shape
+  // a top-k cut above the lists' reach: the chunks' bounds lie around the 64 G-th logit; sixteen times as far below the
+  // maximum, and 40, lies hardly any cut, and the bins from there up are still fine (the smallest value of a row masked
+  // with finite numbers says nothing)
   const uint32_t lmin = wave_min(pl != 0 ? pl : L_NONE);
-  const float xcut = lmin != L_NONE ? fmaxf(xmin, xmax - 4.0f * (xmax - inv_ord32(lmin))) : xmin;
+  const float xcut = lmin != L_NONE ? fmaxf(xmin, xmax - fmaxf(16.0f * (xmax - inv_ord32(lmin)), 40.0f)) : xmin;
   auto leave_open = [&](int how) {
     // 63 bits for the row's mass: at most each chunk's unlisted mass and 1 for every listed logit, times the chunk's maximum
     const double most = wave_sum(pn ? (pp.se + (double)cg) * (double)expf(pm / tt - xs0) : 0.0) * 1.001;
@@ -950,7 +951,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
   const bool cutk = full && top_k > 0 && top_k < n;
   if (Lmax == L_NONE || n == 0 || cutk || (full && (!(tt > 0.0f) || !is_finite(xs0) || !is_finite(xmin / tt)))) {
     const bool plain = full && n > 0 && tt > 0.0f && is_finite(xs0) && is_finite(xmin / tt);
-    leave_open(!plain ? ROW_ANY : !cutk ? ROW_FLAT : top_k <= RCAP ? ROW_TOPK : ROW_ANY);
+    leave_open(!plain ? ROW_ANY : cutk ? ROW_TOPK : ROW_FLAT);
     return;
   }
   // Keys below M are not needed: of a FULL row every key from the largest bound up is listed; a chunk of a TOPK row that
@@ -1411,6 +1412,8 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   const double inv_scale = 1.0 / (double)fsc;
   auto fix_of = [&](float e) -> u64 { return fixed_mass(e, fsh, fsc); };
 
+  u64 Tk = 0, Tfix = 0;  // the smallest key kept by the top-k cut and the mass kept by it (0: not known yet)
+
   VS_TR(A, 1);
   if (how == ROW_FLAT) {
     // ---- one histogram of masses over value bins, one gather of the bins the cuts and the draw can lie in ----
@@ -1691,10 +1694,12 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
     }
     // too many keys in those bins (long runs of tied values): the general method
   } else if (how == ROW_TOPK) {
-    // ---- a top-k cut above the lists' reach: one histogram of counts over value bins, one gather of the bins down to
-    // the one the cut lies in, then workgroup 0 orders the gathered keys by bin and finishes on the k largest. The radix
-    // selects of the general method took nine and more passes for it (top_k 1000, 36 rows of V = 163840 f32: 148 us a
-    // call against 109 in launches of vs_sample_kernel; now 41). ----
+    // ---- a top-k cut above the lists' reach: one histogram of counts over value bins, then one gather. Where the bins
+    // down to the one the cut lies in hold few keys, they are gathered and workgroup 0 orders them by bin and finishes on
+    // the k largest. Otherwise that one bin is gathered and the mass above it summed, and the general method goes on from
+    // the cut's key. The radix selects of the general method took nine and more passes for all of it (36 rows of
+    // V = 163840 f32, top_k 1000: 148 us a call against 109 in launches of vs_sample_kernel, now 41; top_k 5000: 120, 96 and
+    // 82). ----
     const int k = P.top_k;
     const float bsc = xmax > xmin && xmax - xmin < 3.0e38f ? ((float)RNB - 0.5f) / (xmax - xmin) : 0.0f;
     auto bin_of = [&](float x) -> int { return (int)fminf((xmax - x) * bsc, (float)(RNB - 1)); };
@@ -1743,14 +1748,27 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       }
     }
     __syncthreads();
-    const int kb = s.misc[5], ng = kb >= 0 ? s.misc[6] : RCAP + 1;
+    const int kb = s.misc[5], above = kb > 0 ? (int)hc[kb - 1] : 0;
+    const bool all = kb >= 0 && s.misc[6] <= RCAP;
+    const int ng = all ? s.misc[6] : kb >= 0 ? s.misc[6] - above : RCAP + 1;
     if (ng <= RCAP) {
+      const int b0 = all ? 0 : kb;
+      u64 fa = 0;
       tiles_again([&](float x, int id) {
-        if (is_finite(x) & (x >= xmin) && bin_of(x) <= kb) {
-          const int p = atomicAdd(&s.misc[2], 1);
-          if (p < RCAP) s.keys[p] = key64(x, (uint32_t)id);
+        const int bin = is_finite(x) & (x >= xmin) ? bin_of(x) : RNB;
+        if (bin <= kb) {
+          if (bin >= b0) {
+            const int p = atomicAdd(&s.misc[2], 1);
+            if (p < RCAP) s.keys[p] = key64(x, (uint32_t)id);
+          } else {
+            fa += fix_of(mass_at(x / tt - xs0));
+          }
         }
       });
+      if (!all) {
+        fa = block_sum<SNT>(fa, s.red64);
+        if (t == 0) atomicAdd(&o->fix[1], fa);
+      }
       __syncthreads();
       const int nloc = s.misc[2];
       if (t == 0) s.misc[3] = (int)atomicAdd(&o->gcnt, (uint32_t)nloc);
@@ -1762,116 +1780,136 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
         finish();
         return;
       }
-      if (w != 0) return;
+      if (all && w != 0) return;
       u64* mem = (u64*)smem_raw;  // [RCAP] the keys, bin by bin
       u64* srt = mem + RCAP;      // [RCAP] the k largest, in order
       static_assert(2 * RCAP * 8 <= RESOLVE_LDS && RCAP <= 4 * SNT, "both fit the tile area, four keys per thread");
       u64 kr[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) kr[i] = t + i * SNT < ng ? ld_dev(&gkeys[t + i * SNT]) : (u64)0;
+      if (!all) {  // every workgroup: the cut's key, and the mass of the bin's keys from it up
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (kr[i]) mem[atomicAdd(&cur[bin_of(key_value(kr[i]))], 1u)] = kr[i];
-      __syncthreads();
+        for (int i = 0; i < 4; ++i)
+          if (kr[i]) s.keys[t + i * SNT] = kr[i];
+        __syncthreads();
+        u64 f = 0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (kr[i]) {
-          const int bin = bin_of(key_value(kr[i])), end = (int)hc[bin];
-          int r = bin > 0 ? (int)hc[bin - 1] : 0;
-          for (int j = r; j < end; ++j) r += mem[j] > kr[i] ? 1 : 0;
-          if (r < k) srt[r] = kr[i];
+        for (int i = 0; i < 4; ++i) {
+          if (kr[i]) {
+            int r = above;
+            for (int j = 0; j < ng; ++j) r += s.keys[j] > kr[i] ? 1 : 0;
+            if (r < k) f += fix_of(mass_at(key_value(kr[i]) / tt - xs0));
+            if (r == k - 1) s.hk[0] = kr[i];
+          }
         }
+        Tfix = block_sum<SNT>(f, s.red64) + ld_relaxed64(&o->fix[1]);
+        Tk = s.hk[0];
       }
-      __syncthreads();
-      // sampler.py:141-156 on srt[0, k): thread t owns positions E t .. E t + E - 1
-      const int E = (k + SNT - 1) / SNT, i0 = E * t;
-      double pr[4], ls = 0.0, S;
+      if (all) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        pr[q] = q < E && i0 + q < k ? (double)mass_at(key_value(srt[i0 + q]) / tt - xs0) : 0.0;
-        ls += pr[q];
-      }
-      const double base0 = block_scan<SNT>(ls, s.redd, &S) - ls;
-      const double base = base0 / S;
+        for (int i = 0; i < 4; ++i)
+          if (kr[i]) mem[atomicAdd(&cur[bin_of(key_value(kr[i]))], 1u)] = kr[i];
+        __syncthreads();
 #pragma unroll
-      for (int q = 0; q < 4; ++q) pr[q] = pr[q] / S;
-      constexpr int NOWHERE = 1 << 30;
-      int keep = k;
-      uint32_t flags = VS_OUT_COOP;
-      // the first position below `end` whose cumulative mass reaches tgt (NOWHERE: none), its mass and the sum through it
-      // in s.at[0] and s.at[1]
-      auto reach = [&](double tgt, int end) -> int {
-        double c = base, hp = 0.0, hc2 = 0.0;
-        int hit = NOWHERE;
+        for (int i = 0; i < 4; ++i) {
+          if (kr[i]) {
+            const int bin = bin_of(key_value(kr[i])), end = (int)hc[bin];
+            int r = bin > 0 ? (int)hc[bin - 1] : 0;
+            for (int j = r; j < end; ++j) r += mem[j] > kr[i] ? 1 : 0;
+            if (r < k) srt[r] = kr[i];
+          }
+        }
+        __syncthreads();
+        // sampler.py:141-156 on srt[0, k): thread t owns positions E t .. E t + E - 1
+        const int E = (k + SNT - 1) / SNT, i0 = E * t;
+        double pr[4], ls = 0.0, S;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          if (q < E && i0 + q < end) {
-            c += pr[q];
-            if (hit == NOWHERE && c >= tgt) {
-              hit = i0 + q;
-              hp = pr[q];
-              hc2 = c;
-            }
-          }
+          pr[q] = q < E && i0 + q < k ? (double)mass_at(key_value(srt[i0 + q]) / tt - xs0) : 0.0;
+          ls += pr[q];
         }
-        const int at = block_min<SNT>(hit, s.red);
-        if (at != NOWHERE && at == hit) {
-          s.at[0] = hp;
-          s.at[1] = hc2;
-        }
-        __syncthreads();
-        return at;
-      };
-      // the position `at` itself: its mass and the sum through it, likewise
-      auto look = [&](int at) {
-        if (at / E == t) {
-          double c = base, hp = 0.0;
+        const double base0 = block_scan<SNT>(ls, s.redd, &S) - ls;
+        const double base = base0 / S;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) pr[q] = pr[q] / S;
+        constexpr int NOWHERE = 1 << 30;
+        int keep = k;
+        uint32_t flags = VS_OUT_COOP;
+        // the first position below `end` whose cumulative mass reaches tgt (NOWHERE: none), its mass and the sum through it
+        // in s.at[0] and s.at[1]
+        auto reach = [&](double tgt, int end) -> int {
+          double c = base, hp = 0.0, hc2 = 0.0;
+          int hit = NOWHERE;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            if (q < E && i0 + q <= at) {
+            if (q < E && i0 + q < end) {
               c += pr[q];
-              hp = pr[q];
+              if (hit == NOWHERE && c >= tgt) {
+                hit = i0 + q;
+                hp = pr[q];
+                hc2 = c;
+              }
             }
           }
-          s.at[0] = hp;
-          s.at[1] = c;
+          const int at = block_min<SNT>(hit, s.red);
+          if (at != NOWHERE && at == hit) {
+            s.at[0] = hp;
+            s.at[1] = hc2;
+          }
+          __syncthreads();
+          return at;
+        };
+        // the position `at` itself: its mass and the sum through it, likewise
+        auto look = [&](int at) {
+          if (at / E == t) {
+            double c = base, hp = 0.0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              if (q < E && i0 + q <= at) {
+                c += pr[q];
+                hp = pr[q];
+              }
+            }
+            s.at[0] = hp;
+            s.at[1] = c;
+          }
+          __syncthreads();
+        };
+        if (has_tp) {  // :145-148
+          const int at = reach(P.top_p, k);
+          if (at != NOWHERE) {
+            keep = at + 1;
+            if (fabs(s.at[1] - P.top_p) < 1e-6 || fabs(s.at[1] - s.at[0] - P.top_p) < 1e-6)
+              flags |= VS_OUT_TOPP_BOUNDARY;
+          }
+        }
+        if (has_mp) {  // :149-152 (the largest key's mass is 1 before the division by S)
+          const double pthr = (1.0 / S) * P.min_p;
+          int hit = NOWHERE;
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (hit == NOWHERE && q < E && i0 + q < k && pr[q] < pthr) hit = i0 + q;
+          const int at = block_min<SNT>(hit, s.red);
+          const int cnt = at == NOWHERE ? k : max(at, 1);
+          keep = cnt < keep ? cnt : keep;
         }
         __syncthreads();
-      };
-      if (has_tp) {  // :145-148
-        const int at = reach(P.top_p, k);
-        if (at != NOWHERE) {
-          keep = at + 1;
-          if (fabs(s.at[1] - P.top_p) < 1e-6 || fabs(s.at[1] - s.at[0] - P.top_p) < 1e-6)
-            flags |= VS_OUT_TOPP_BOUNDARY;
-        }
+        look(keep - 1);
+        const double z = s.at[1], uz = P.u * z;  // :153-154
+        __syncthreads();
+        int j = reach(uz, keep);
+        if (j == NOWHERE) look(j = keep - 1);  // :155-156
+        const double hp = s.at[0], hs = s.at[1], tol = 1e-6 * z;
+        if (fabs(hs - uz) < tol || (j >= 1 && fabs(hs - hp - uz) < tol)) flags |= VS_OUT_DRAW_BOUNDARY;
+        fin.token = (int32_t)key_index(srt[j]);
+        fin.lp = (float)log_ratio(hp, z);
+        fin.keep = keep;
+        fin.flags = flags;
+        finish();
+        return;
       }
-      if (has_mp) {  // :149-152 (the largest key's mass is 1 before the division by S)
-        const double pthr = (1.0 / S) * P.min_p;
-        int hit = NOWHERE;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (hit == NOWHERE && q < E && i0 + q < k && pr[q] < pthr) hit = i0 + q;
-        const int at = block_min<SNT>(hit, s.red);
-        const int cnt = at == NOWHERE ? k : max(at, 1);
-        keep = cnt < keep ? cnt : keep;
-      }
-      __syncthreads();
-      look(keep - 1);
-      const double z = s.at[1], uz = P.u * z;  // :153-154
-      __syncthreads();
-      int j = reach(uz, keep);
-      if (j == NOWHERE) look(j = keep - 1);  // :155-156
-      const double hp = s.at[0], hs = s.at[1], tol = 1e-6 * z;
-      if (fabs(hs - uz) < tol || (j >= 1 && fabs(hs - hp - uz) < tol)) flags |= VS_OUT_DRAW_BOUNDARY;
-      fin.token = (int32_t)key_index(srt[j]);
-      fin.lp = (float)log_ratio(hp, z);
-      fin.keep = keep;
-      fin.flags = flags;
-      finish();
-      return;
     }
-    // more keys than are gathered (tied values, a row of an odd shape): the general method, once everyone has read the sums
+    // the general method, once everyone has read the sums
     if (!barrier()) {
       finish();
       return;
@@ -1910,7 +1948,6 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
   }
   int k = P.top_k > 0 ? (P.top_k < n ? P.top_k : n) : n;  // sampler.py:133-134
   if (k < 1) k = 1;
-  u64 Tk = 0;  // the smallest key kept by the top-k cut
   const bool cutk = k < n;
   const float kthr = cutk ? -__builtin_inff() : thr;
   auto kept = [&](float x, int id, u64& key, float& xs) -> bool {
@@ -1985,7 +2022,7 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
       }
     }
   };
-  if (cutk) {
+  if (cutk && Tk == 0) {
     const Sel sk = select(true, (u64)k);
     if (!ok) {
       finish();
@@ -2016,12 +2053,12 @@ __global__ __launch_bounds__(SNT, 2) void vs_resolve_kernel(SampleArgs A) {
     }
     return barrier();
   };
-  if (!sums(0.0, 0.0, 1)) {
+  if (Tfix == 0 && !sums(0.0, 0.0, 1)) {
     finish();
     return;
   }
-  const u64 Sfix = ld_relaxed64(&o->fix[1]);
-  int keep = (int)ld_relaxed(&o->cnt[2]);
+  const u64 Sfix = Tfix ? Tfix : ld_relaxed64(&o->fix[1]);
+  int keep = Tfix ? k : (int)ld_relaxed(&o->cnt[2]);
   u64 zfix = Sfix;
   uint32_t flags = VS_OUT_COOP;  // the general kernel's route bit
   if (has_tp) {  // sampler.py:145-148

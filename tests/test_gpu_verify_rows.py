@@ -152,3 +152,21 @@ def test_graph_replays_between_other_calls(dev):
         assert torch.equal(verify_greedy(few, fd, V).argmax, want_few)
         torch.cuda.synchronize()
         check(o, x, drafts.cpu().numpy(), V, i)
+
+
+@pytest.mark.parametrize("dtype,line", [(torch.float32, 4 << 20), (torch.bfloat16, 2 << 20), (torch.float16, 3 << 20)])
+@pytest.mark.parametrize("V", [16381, 100003, 8193])
+def test_unaligned_rows_around_the_line(dev, dtype, line, V):
+    """Few unaligned rows take the one-launch kernel below a number of logits and the two launches from there on (rows
+    that fill their workgroups badly keep to the first): both give the oracle's answer."""
+    for n in (line // V, line // V + 1):
+        T = 3
+        B = -(-n // T)
+        x = block(dev, B, T, V, V, 0, dtype, n)
+        tok = x.float().argmax(-1).cpu().numpy()
+        drafts = tok[:, :-1].astype(np.int32).copy()
+        drafts[::2, 1] += 1
+        print(f"[line] {dtype} V={V} B={B} T={T}", flush=True)
+        o = verify_greedy(x, torch.from_numpy(drafts).to(dev), V)
+        torch.cuda.synchronize()
+        check(o, x, drafts, V, (dtype, V, n))

@@ -759,12 +759,17 @@ extern "C" int vs_verify_greedy(const void* logits, int dtype, int B, int T, int
   // launches, each with its own start, tail and finish, took for 272 rows of V = 248320 bf16 53.8 us, the two take 32.3;
   // V = 163840: 37.0 and 21.5 in bf16, 54.6 and 35.8 in f32. In one launch vs_verify_kernel is the better one (17 rows of
   // V = 163840 bf16: 6.8 us against 8.5; 102 rows 13.5 against 13.4), except where rows are unaligned, since it reads
-  // those element by element: 17 rows of ld = 163843 9.9 against 8.8, 68 rows 19.9 against 12.4, 68 of 50003 f16 11.2
-  // against 10.1, but 34 of those 8.7 against 9.7. Hence the line at 2 M logits.
+  // those element by element. One launch / the two on unaligned rows, by the logits of the call: bf16 2.2 M (68 rows of
+  // 32001) 11.0 / 10.2, 2.8 M (17 of 163843) 11.0 / 10.0; f16 2.2 M 11.1 / 11.7, 2.6 M (51 of 50003) 10.2 / 11.3, 2.8 M
+  // 11.1 / 11.4, 3.4 M (34 of 100003) 13.5 / 11.3; f32 2.6 M 9.3 / 9.8, 2.8 M 9.2 / 9.5, 4.2 M (68 of 61441) 10.2 / 10.8,
+  // (17 of 248323) 10.7 / 10.7, 5.6 M (34 of 163843) 12.4 / 11.1. Hence the lines at 2, 3 and 4 M logits; f16 too at
+  // 4 M where a row leaves a third of its workgroups' places empty (8193: 510 rows 11.3 / 12.1, 527 13.8 / 13.3).
   const int es = 16 / VEC;
   const int span = vocab_valid + (ld % VEC == 0 ? (int)((uintptr_t)logits % 16) / es : VEC - 1);
   const int tile = VNT * vs_lane_logits(dtype), gs = (span + tile - 1) / tile;
-  const bool many = R > rpl || (!a.vec_ok && (int64_t)R * vocab_valid >= (2 << 20));
+  const bool full = 3 * (int64_t)span >= 2 * (int64_t)gs * tile;
+  const int line = (dtype == VS_BF16 ? 2 : dtype == VS_F16 && full ? 3 : 4) << 20;
+  const bool many = R > rpl || (!a.vec_ok && (int64_t)R * vocab_valid >= line);
   if (many && gs <= VGMAX && (uintptr_t)logits % es == 0) {
     a.CH = ((span + gs - 1) / gs + VEC - 1) / VEC * VEC;
     a.G = (span + a.CH - 1) / a.CH;

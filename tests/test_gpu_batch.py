@@ -312,3 +312,40 @@ def test_open_rows_repeat_bit_for_bit(dev, kind):
     first = ops.sample_rows(xt, rows).block.clone()
     for _ in range(12):
         assert torch.equal(ops.sample_rows(xt, rows).block, first)
+
+
+@pytest.mark.parametrize("down", [8.0, 10.0, 12.0])
+def test_mass_of_the_unlisted_logits(dev, down):
+    """Requests without a cut that draw a listed token: the logprob is the logarithm of the row's mass, half of it in
+    tied logits far below the maximum that no list holds, at the temperatures where (x - max) (log2 e / t) in float32 is
+    furthest from the quotients' difference. Each mass is within 2 ulp of its exponential (2.4e-7), a tree of four adds 2
+    halves of an ulp (1.2e-7), on at most 0.55 of the mass; the float32 logarithm and the result add an ulp of the logprob
+    (below 1) each: 0.55 * 3.6e-7 + 1.0e-7 = 3.0e-7 in all, for every temperature."""
+    rng = np.random.default_rng(int(down))
+    B, V = 66, 163840
+    f = np.float32
+    ts = rng.uniform(0.6, 1.4, 100000).astype(f)
+    x0 = f(5) - f(down) * ts
+    folded = np.exp2(((x0 - f(5)) * (f(np.log2(np.e)) / ts)).astype(np.float64))
+    ts = ts[np.argsort(-np.abs(folded / np.exp((x0 / ts).astype(np.float64) - f(5) / ts) - 1))[:B]]
+    x = np.empty((B, V), np.float32)
+    for r in range(B):  # a maximum of 5, a floor whose mass is about 1, logits above it to list, the rest near nothing
+        x[r] = 5.0 - 38.0 * ts[r]
+        at = rng.permutation(V)
+        x[r, at[:min(int(np.exp(down)), V - V // 50)]] = f(5) - f(down) * ts[r]
+        x[r, at[V - V // 60:]] = 5.0 - ts[r] * (down - 0.5 - 0.3 * rng.random(V // 60))
+        x[r, at[V - V // 60 - 1]] = 5.0
+    rows = ops.pack_rows([Sampling(temperature=float(t)) for t in ts], np.full(B, 1e-9), V).to(dev)
+    print(f"[mass] {down}", flush=True)
+    o = ops.sample_rows(torch.from_numpy(x).to(dev), rows)
+    lp = o.logprobs.cpu().numpy().astype(np.float64)
+    assert np.array_equal(o.ids.cpu().numpy(), x.argmax(1))
+    assert np.all(o.keep.cpu().numpy() == V)
+    done = ops.workspace(dev, 64 * _lib.load().vs_sample_workspace_bytes(1, V))[64:64 + 56]  # the rows' open flags
+    assert int(done.sum()) == 0  # finished from the lists
+    xs = x / ts[:, None]  # float32, as the sampler divides
+    d = xs.astype(np.float64) - xs.max(1, keepdims=True)
+    want = -np.log(np.where(d >= -40.0, np.exp(d), 0.0).sum(1))
+    err = np.abs(lp - want)
+    print(f"[mass] largest error {err.max():.2e}, mean {np.mean(lp - want):.2e}", flush=True)
+    assert err.max() <= 3.0e-7

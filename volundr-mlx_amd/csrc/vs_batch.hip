@@ -722,15 +722,24 @@ __global__ __launch_bounds__(SNT, 4) void vs_batch_kernel(SampleArgs A) {
   };
   double rest = 0.0;
   if (full && nf > 0) {
-    const float c = L2E / P.temperature;
-    float a4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    // x/t rounded as in sampler.py:141, by the rounded reciprocal and the quotient's remainder; its exponential to 2 ulp
+    // (exp_nonpos); four of them at a time added as a tree, then float64. With (x - max) (log2 e / t) in the exponent and
+    // sums of eight the mass was off by up to 1e-6 for tied values 15 to 20 nats down, and all to one side for some t.
+    const float tt = P.temperature, rt = 1.0f / tt, xw = wm / tt, low = wm - 150.0f * tt;
 #pragma unroll
-    for (int i = 0; i < E; ++i) {
-      const bool in = v[i] >= Lf;
-      a4[i % 4] += __builtin_amdgcn_exp2f(in ? -__builtin_inff() : (v[i] - wm) * c);
-      stage(i, in);
+    for (int i0 = 0; i0 < E; i0 += 4) {
+      float e[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float x = v[i0 + j], q = x * rt;
+        const bool in = x >= Lf;
+        const float m = exp_nonpos(__builtin_fmaf(__builtin_fmaf(-q, tt, x), rt, q) - xw);
+        e[j] = !in & (x > low) ? m : 0.0f;
+        stage(i0 + j, in);
+      }
+      rest += (double)((e[0] + e[1]) + (e[2] + e[3]));
     }
-    rest = wave_sum_dpp(((double)a4[0] + (double)a4[1]) + ((double)a4[2] + (double)a4[3]));
+    rest = wave_sum_dpp(rest);
   } else {
 #pragma unroll
     for (int i = 0; i < E; ++i) stage(i, v[i] >= Lf);
@@ -963,7 +972,11 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
   float xq = -__builtin_inff();
   if (has_mp) xq = P.min_p < 1.0 ? xmax + tt * (logf((float)P.min_p) - 1e-4f - 1e-5f * fabsf(xs0)) : xmax;
   // FULL: the mass of the unlisted logits, relative to the row's maximum
-  const double rsum = full ? wave_sum(pn && pp.se > 0.0 ? pp.se * (double)expf(pm / tt - xs0) : 0.0) : 0.0;
+  // (the chunk's scale e^(pm/tt - xs0) with the difference's rounding made good: it is common to all of the chunk)
+  const double dm = (double)(pm / tt) - (double)xs0;
+  const float dmf = (float)dm;
+  const double rsum =
+      full ? wave_sum(pn && pp.se > 0.0 ? pp.se * ((double)expf(dmf) * (1.0 + (dm - (double)dmf))) : 0.0) : 0.0;
   if (full && !(has_mp && xq > xlow)) {
     // a flat row shows here: no listed logit's mass is above 1, so the lists cannot hold the share that is asked for
     const double p = P.top_p < 1.0 ? P.top_p : (has_mp ? 1.0 : P.u);

@@ -349,3 +349,26 @@ def test_mass_of_the_unlisted_logits(dev, down):
     err = np.abs(lp - want)
     print(f"[mass] largest error {err.max():.2e}, mean {np.mean(lp - want):.2e}", flush=True)
     assert err.max() <= 3.0e-7
+
+
+def test_logprobs_have_no_bias(dev):
+    """Nucleus rows of a language model's shape: the logprob is the float32 difference the reference takes less the
+    logarithm of the kept mass, rounded once. Masses (2 ulp), the logarithm and the result (an ulp of a few units) leave
+    a row's error within about 2.5e-7 of no preferred sign, so the mean over 128 rows within 3 * 2.5e-7 / sqrt(128)."""
+    rng = np.random.default_rng(31)
+    B, V, n = 128, 32768, 900
+    ts = rng.uniform(0.6, 1.1, B).astype(np.float32)
+    x = (rng.standard_normal((B, V)) * 2).astype(np.float32)
+    for r in range(B):
+        x[r, rng.choice(V, n, replace=False)] = (16.0 - rng.random() * 0.6 * np.arange(n) ** 0.4
+                                                 + 0.3 * rng.standard_normal(n)).astype(np.float32)
+    ps = [Sampling(temperature=float(t), top_p=0.8) for t in ts]
+    u = rng.random(B)
+    print("[bias] 128 rows", flush=True)
+    o = sample_batch(torch.from_numpy(x).to(dev), ps, u)
+    refs = [S.sample(x[r], ps[r], float(u[r])) for r in range(B)]
+    check_sample(o, refs, "logprobs", 1)
+    lp, ids, keep = (t.cpu().numpy() for t in (o.logprobs, o.ids, o.keep))
+    err = [float(lp[r]) - f.logprob for r, f in enumerate(refs) if ids[r] == f.token and keep[r] == f.keep]
+    print(f"[bias] mean {np.mean(err):.2e}, largest {np.max(np.abs(err)):.2e}", flush=True)
+    assert abs(np.mean(err)) <= 3 * 2.5e-7 / np.sqrt(B)

@@ -852,7 +852,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_batch_kernel(SampleArgs A) {
 struct FinishLds {
   uint32_t hc[NBIN];  // counts by value bin
   uint32_t at[NBIN];  // the next place of each bin
-  double hf[NBIN];    // masses
+  u64 hf[NBIN];       // masses, in fixed point (at 2^50): the same sums in any order
   u64 sel[BSEL];      // the keys to rank
   u64 tk[BSEL];       // ranked
   double sum[NRED];
@@ -874,7 +874,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
   const Part pp = parts[ln < G ? ln : 0];
   if (t < NBIN) {
     s.hc[t] = 0;
-    s.hf[t] = 0.0;
+    s.hf[t] = 0;
   }
   if (t == 0) s.misc[4] = 0;
   RowIn R;
@@ -1033,7 +1033,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
       if (kk[u] >= M) {
         const int b = bin_of(x);
         atomicAdd(&s.hc[b], 1u);
-        if (full) unsafeAtomicAdd(&s.hf[b], (double)e);
+        if (full) atomicAdd(&s.hf[b], fixed_mass(e, 0x1p18f, 0x1p50f));
       } else {
         kk[u] = 0;
       }
@@ -1070,9 +1070,9 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
   bool mend = false;  // every key past the cut bin fails min-p
   {
     int c4[4];
-    double f4[4];
+    u64 f4[4];
     int lc = 0;
-    double lf = 0.0;
+    u64 lf = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       c4[i] = (int)s.hc[4 * ln + i];
@@ -1081,9 +1081,9 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
       lf += f4[i];
     }
     const int ic = wave_scan(lc);
-    const double iff = wave_scan(lf);
+    const u64 iff = wave_scan(lf);
     int cc = ic - lc;
-    double cf = iff - lf;
+    u64 cf = iff - lf;
     // the bin where the count reaches keff (TOPK), or the mass reaches the top-p cut, else the draw (FULL)
     const bool cuts = P.top_p < 1.0 || P.min_p > 0.0;
     const double tgt = P.top_p < 1.0 ? P.top_p * S : (cuts ? 1e300 : P.u * S * (1.0 + 1e-12));
@@ -1093,7 +1093,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
       cc += c4[i];
       cf += f4[i];
       cum[i] = cc;
-      if (hit == 1 << 20 && c4[i] > 0 && (full ? cf >= tgt : cc >= keff)) hit = 4 * ln + i;
+      if (hit == 1 << 20 && c4[i] > 0 && (full ? (double)cf * 0x1p-50 >= tgt : cc >= keff)) hit = 4 * ln + i;
       if (t < WAVE) s.at[4 * ln + i] = (uint32_t)(cc - c4[i]);
     }
     cut = wave_min(hit);

@@ -559,7 +559,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_batch_kernel(SampleArgs A) {
   Part* part = (Part*)part_area(A.ws, row) + g;
   u64* list = (u64*)list_area(A.ws, row) + (size_t)g * A.kcap;
   const int l0 = p0 - R.mis;
-  const float L2E = 1.44269504088896340736f;
+  constexpr float L2E = 1.44269504088896340736f;
   // the lane's largest value, and whether it holds a NaN or an infinity (x * 0 is NaN then)
   float best = -__builtin_inff(), zero[2] = {0.0f, 0.0f};
 #pragma unroll
@@ -727,9 +727,10 @@ __global__ __launch_bounds__(SNT, 4) void vs_batch_kernel(SampleArgs A) {
   double rest = 0.0;
   if (full && nf > 0) {
     // x/t rounded as in sampler.py:141, by the rounded reciprocal and the quotient's remainder; its exponential to 2 ulp
-    // (exp_nonpos); four of them at a time added as a tree, then float64. With (x - max) (log2 e / t) in the exponent and
+    // (as exp_nonpos); four of them at a time added as a tree, then float64. With (x - max) (log2 e / t) in the exponent and
     // sums of eight the mass was off by up to 1e-6 for tied values 15 to 20 nats down, and all to one side for some t.
-    const float tt = P.temperature, rt = 1.0f / tt, xw = wm / tt, low = wm - 150.0f * tt;
+    const float tt = P.temperature, rt = 1.0f / tt, xw = wm / tt, low = -150.0f;
+    constexpr float L2E_LO = 1.9259629891e-8f;  // log2(e) less L2E
 #pragma unroll
     for (int i0 = 0; i0 < E; i0 += 4) {
       float e[4];
@@ -737,8 +738,11 @@ __global__ __launch_bounds__(SNT, 4) void vs_batch_kernel(SampleArgs A) {
       for (int j = 0; j < 4; ++j) {
         const float x = v[i0 + j], q = x * rt;
         const bool in = x >= Lf;
-        const float m = exp_nonpos(__builtin_fmaf(__builtin_fmaf(-q, tt, x), rt, q) - xw);
-        e[j] = !in & (x > low) ? m : 0.0f;
+        // (a NaN, from an x of -inf, becomes the lower limit, whose mass is a float zero)
+        const float d = max3f(__builtin_fmaf(__builtin_fmaf(-q, tt, x), rt, q) - xw, low, low);
+        const float y = d * L2E, yl = __builtin_fmaf(d, L2E_LO, __builtin_fmaf(d, L2E, -y));
+        const float m = __builtin_amdgcn_exp2f(y);
+        e[j] = in ? 0.0f : __builtin_fmaf(m, yl * 0.693147180559945309f, m);
         stage(i0 + j, in);
       }
       rest += (double)((e[0] + e[1]) + (e[2] + e[3]));

@@ -382,8 +382,9 @@ __device__ __forceinline__ float mass_at(float d) { return exp_nonpos(fmaxf(d, -
 
 // sampler.py:144-156 on the n largest keys of a row, sorted descending in LDS, where S is the mass of the row's whole
 // kept set (n <= 64 * EM keys reach past every cut: see the merge). `total` is the size of the kept set, -1 where it is
-// not known (then top-p or min-p cuts it); `mend`: every key of the row past these n fails min-p. Lane layout and order of sums as in wave_sample_em. Lane 0 leaves token,
-// keep, flags and logprob in LDS, misc[0] = 0 if a cut or the draw was not found among the keys after all.
+// not known (then top-p or min-p cuts it); `mend`: every key of the row past these n fails min-p. Lane layout and order
+// of sums as in wave_sample_em. Lane 0 leaves token, keep, flags and logprob in LDS, misc[0] = 0 if a cut or the draw was
+// not found among the keys after all.
 template <int EM>
 __device__ __forceinline__ void wave_sample_tail(const u64* a, int n, double S, int total, bool mend,
                                                  const vs_row_params& P, int* misc, double* lp) {
@@ -509,7 +510,7 @@ __device__ __forceinline__ void wave_sample_tail(const u64* a, int n, double S, 
 
 // ---------------------------------------------------------------------------------------------------------------
 // Pass over the logits. What bounds it: the chain load - edits - bound - list of each workgroup with two or three of
-// them per CU (128 mixed requests at V = 163840 fp32: 31.9 us for 84 MB, 2.6 TB/s; the vector instructions alone would
+// them per CU (128 mixed requests at V = 163840 fp32: 32.8 us for 84 MB, 2.6 TB/s; the vector instructions alone would
 // take 12 us). Nothing waits on anything outside the workgroup, and the lists travel by plain stores: with the merge in
 // the row's last workgroup instead of a launch of its own this kernel took 52 us (arrivals, 128 merges of 11 us each in
 // workgroups that hold stream slots, and an XCD a little behind the others arriving last in every row and so getting
@@ -849,8 +850,8 @@ __global__ __launch_bounds__(SNT, 4) void vs_batch_kernel(SampleArgs A) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// One workgroup per row finishes it from the lists, or leaves it open. A chain of small steps (8 us for top-k rows, 14 us
-// with FULL rows among 128 mixed ones): the loads, value bins over the keys, the cut bin, the keys down to it ranked, the
+// One workgroup per row finishes it from the lists, or leaves it open. A chain of small steps (8 us for top-k rows, 12.6
+// us with FULL rows among 128 mixed ones): the loads, value bins over the keys, the cut bin, the keys down to it ranked, the
 // draw in one wave.
 // ---------------------------------------------------------------------------------------------------------------
 struct FinishLds {
@@ -1237,7 +1238,7 @@ __global__ __launch_bounds__(SNT, 4) void vs_finish_kernel(SampleArgs A) {
 // pass. All of them see the same sums and take the same decisions; workgroup 0 writes the result. A wait that reaches its
 // bound ends the workgroup; workgroup 0 then reports VS_OUT_TIMEOUT (it passes a barrier only when every workgroup has
 // contributed to everything before it). Where a workgroup's share of the row fits LDS the second pass of the flat method
-// reads it there (24576 logits; 20 near-flat rows of V = 163840: 53 us per call, 60 in two launches of vs_sample_kernel).
+// reads it there (24576 logits; 20 near-flat rows of V = 163840: 39 us per call, 56 in two launches of vs_sample_kernel).
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int RE = 16;                          // logits per lane and tile
 constexpr int RTILE = RE * SNT;                 // positions per tile at most

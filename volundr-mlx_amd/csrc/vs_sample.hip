@@ -2814,11 +2814,18 @@ static int sample_launch(const void* logits, int dtype, int B, int V, int64_t ld
   a.trace = g_trace;
   // A batch that takes more than one launch here goes to vs_batch_kernel instead. One launch of this kernel is the
   // shorter way for up to RB rows unless their mix is unlucky (V = 163840 fp32, us per call here / there: 16 top-k rows
-  // 13 / 18, 16 near-flat ones 31 / 48, 16 mixed requests 61 / 26), a chain of launches is not (20 / 64 rows: top-k
-  // 27 / 19 and 55 / 22, near-flat 60 / 51 and 127 / 108, mixed requests 140 / 27 and 255 / 37). Rows below 8192
-  // logits give its workgroups too few lanes to bound their lists with. The testing flags (but the exchange level, which
-  // that route has only one of) and cooperative launches concern this kernel's waits, and vs_sample_batch_noalloc's
-  // scratch rows are its own.
+  // 13 / 18, 16 near-flat ones 31 / 48, 16 mixed requests 61 / 26). A chain of launches is not, at its worst (20 rows, the
+  // second launch nearly empty), its best (36 rows, two full launches) and beyond (64 rows):
+  //                  20        36        64                        20        36        64
+  //   top-k 20    27 / 19   28 / 21   57 / 23      nucleus      58 / 23  110 / 26  119 / 31
+  //   top-k 200   81 / 29   85 / 33  171 / 30      min-p       146 / 23  141 / 26  291 / 31
+  //   top-k 256   90 / 30   95 / 34  182 / 37      no cut       56 / 45   60 / 54  118 / 66
+  //   top-k 1000 107 / 35  108 / 43  198 / 60      near-flat    56 / 39   63 / 47  127 / 66
+  //   top-k 5000  88 / 63   96 / 82  185 / 130     greedy       18 / 12   20 / 12   40 / 16
+  // Closest where rows without a cut are many and short: V = 32768, 128 rows 43.0 / 43.6; V = 8192, 37.0 / 35.3. Rows
+  // below 8192 logits give its workgroups too few lanes to bound their lists with. The testing flags (but the exchange
+  // level, which that route has only one of) and cooperative launches concern this kernel's waits, and
+  // vs_sample_batch_noalloc's scratch rows are its own.
   const size_t ws_rows = ws_bytes / ROW_WS;
   if (B > RB && V >= 8192 && list_k <= WAVE && rows_cap == RPL_MAX && !coop && !(g_debug & ~VS_DEBUG_NO_XCD_EXCHANGE) &&
       (uintptr_t)logits % (16 / VEC) == 0)
